@@ -34,82 +34,9 @@
 #include <vector>
 
 #include "bamhip_internal.h"
-
-// Contraction of a*b + c into an FMA only within one source expression: the
-// fused operations are then fixed by the source, not by per-kernel backend
-// choices, so every instantiation of the tile kernel (tile shape, staging,
-// register budget) rounds identically and gives bitwise the same RHS.
-#pragma clang fp contract(on)
-
-// compile-time loop: f(integral_constant<int, I>) for I = 0..N-1; used for
-// loops whose body holds a barrier, which the compiler does not unroll, so
-// that per-field arrays keep constant indices and stay in registers
-template <class F, int... I>
-__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F &&f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
+#include "z4c_tile.h"
 
 namespace bamhip {
-
-// u: the state the stencils read; r: output (the RHS, unew = upre + c RHS, or
-// in an RK4 stage the next stage's state); p: upre, or the RK4 step's start
-// state in a stage.  In an RK4 stage (read and written at the point only):
-// a: the accumulator read, c: the accumulator written (c = a + wc RHS), cp:
-// where the start state p is copied to (or unused).
-struct Z4cPtrs {
-  const double *u[BAMHIP_Z4C_NVARS];
-  double *r[BAMHIP_Z4C_NVARS];
-  const double *p[BAMHIP_Z4C_NVARS];
-  double *c[BAMHIP_Z4C_NVARS];
-  const double *a[BAMHIP_Z4C_NVARS];
-  double *cp[BAMHIP_Z4C_NVARS];
-};
-
-struct Z4cGeo {
-  int m, n, o;      // box points
-  long noffset;
-  int lo[3], hi[3]; // computed index range [lo, hi] per direction
-  long sj, sk;      // strides (di = 1)
-  double h[3], ih[3];
-  double i12h[3], i12hh[3], i144hh[3];  // 4th order: 1/(12h), 1/(12h^2), mixed 1/(144 ha hb) (xy, xz, yz)
-  double i2h[3], ihh[3], i4hh[3];       // 2nd order: 1/(2h), 1/h^2, mixed 1/(4 ha hb)
-  int edge_only;    // Edge kernel: skip points that the bulk kernel computes
-};
-
-struct Z4cK {
-  int order_centered, order_advection, lopsided, order_dissipation;
-  double dissfactor, kappa1, kappa2, zeroThetaRHS;
-  int subtractA, normalizedetg;
-  double oploglapse, oploglapse2, oplogwithshift, harmoniclapse, lapseharmonicf;
-  double gamma0factor, gamma2factor, withGadv, withShiftadv, withBadv, withB;
-  double shiftalphapower, shiftgammacoeff, shiftdriver;
-  double chiDivFloor, chipsipower;
-  double c;
-  int addlinear;
-  // RK4 stage (rk.c:231-252) fused into the store: c = a + wc RHS, when
-  // has_v r = p + wv RHS, when has_cp cp = p
-  int rk, has_v, has_cp;
-  double wc, wv;
-};
-
-// scheduling fence: keeps the machine scheduler from hoisting the loads of
-// later derivative groups above earlier ones, which would keep hundreds of
-// FP64 stencil values live at once and spill
-#define BH_PHASE() __builtin_amdgcn_sched_barrier(0)
-
-// index of component (a,b) in xx xy xz yy yz zz storage; closed form (not
-// recursive) so that it folds to a constant once the loops are unrolled and
-// every tensor array stays in registers
-__device__ __forceinline__ constexpr int sy(int a, int b) {
-  return (a < b ? a : b) * (5 - (a < b ? a : b)) / 2 + (a < b ? b : a);
-}
-__device__ __forceinline__ constexpr int mixid(int a, int b) {  // xy=0 xz=1 yz=2
-  return (a + b) - 1;
-}
 
 // ---------------------------------------------------------------- providers
 // lop-sided advection rows: stencil4[offset] of order 4 and the order-2 rows
@@ -584,867 +511,6 @@ __device__ __forceinline__ bool z4c_point(D &dv, const Z4cPtrs &P, const Z4cK &K
   return finite;
 }
 
-// ------------------------------------------------------- bulk kernel (LDS)
-// Output tile of TX x TY x TZ points per block (256 threads, one point per
-// thread).  Each of the 25 grid functions is staged in turn into an LDS tile
-// with a halo of 3 points (the reach of the lop-sided advection stencil), so
-// every stencil neighbour is an immediate-offset ds_read_b64 from one
-// per-thread LDS address.  The algebra is ordered by staged field: each
-// field's derivatives, advection and dissipation are consumed as soon as the
-// field is in LDS.  The bulk uses 16 x 4 x 4 tiles (long x rows for
-// coalesced loads); the box-edge shell, two points thick, uses slabs of
-// 2 x 16 x 8, 16 x 2 x 8 and 16 x 8 x 2 on the x, y and z faces.
-constexpr int HALO = 3;
-constexpr int NTHR = 256;
-// PX: unused LDS columns at the end of each tile row (the row stride SX is
-// the staged width WX plus PX), chosen so that the 16 lanes of a read phase
-// fall on distinct banks
-// ORD: which point of the tile thread t of the block computes (64 threads
-// form a wave): 0, x fastest, then y, then z; 1, y fastest, then z, then x
-// (a wave keeps one x, as the layers of an x-face slab do); 2, x fastest,
-// then z, then y (a wave keeps one y).
-template <int TX_, int TY_, int TZ_, int PX = 0, int ORD = 0>
-struct Lay {
-  static constexpr int TX = TX_, TY = TY_, TZ = TZ_;
-  static constexpr int WX = TX + 2 * HALO;
-  static constexpr int SX = WX + PX, SY = TY + 2 * HALO, SZ = TZ + 2 * HALO;
-  static constexpr int TILE = SX * SY * SZ;
-  static constexpr int NLOAD = (TILE + NTHR - 1) / NTHR;
-  static_assert(TX * TY * TZ == NTHR, "one point per thread");
-  static_assert(ORD >= 0 && ORD <= 2, "thread order");
-  __device__ static void coords(int t, int &x, int &y, int &z) {
-    if constexpr (ORD == 1) {
-      y = t % TY;
-      z = (t / TY) % TZ;
-      x = t / (TY * TZ);
-    } else if constexpr (ORD == 2) {
-      x = t % TX;
-      z = (t / TX) % TZ;
-      y = t / (TX * TZ);
-    } else {
-      x = t % TX;
-      y = (t / TX) % TY;
-      z = t / (TX * TY);
-    }
-  }
-};
-using LBulk = Lay<16, 4, 4>;
-// x faces: rows of 2 points, so without padding (stride 8 doubles) the
-// lanes (x, y) = (0..1, 0..7) of a read phase meet on 4 banks; a stride of 10
-// spreads them over all 32
-using LSlabX = Lay<2, 16, 8, 2>;
-using LSlabY = Lay<16, 2, 8>;
-using LSlabZ = Lay<16, 8, 2>;
-using LLayX = Lay<1, 16, 16>;
-using LLayY = Lay<16, 1, 16>;
-using LLayZ = Lay<16, 16, 1>;
-
-// a thread's tile corner in the LDS tile of layout L (its point is at +HALO)
-template <class L>
-struct TP {
-  const double *p;
-};
-
-template <int DX, int DY, int DZ, class L>
-__device__ __forceinline__ double at(TP<L> T) {
-  return T.p[(DX + HALO) + L::SX * ((DY + HALO) + L::SY * (DZ + HALO))];
-}
-// neighbour at offset o along direction A
-template <int A, int O, class L>
-__device__ __forceinline__ double ax(TP<L> T) {
-  return at<(A == 0 ? O : 0), (A == 1 ? O : 0), (A == 2 ? O : 0)>(T);
-}
-template <int A, class L>
-__device__ __forceinline__ double t_d1(TP<L> T, const Z4cGeo &G) {
-  return ((ax<A, -2>(T) - ax<A, 2>(T)) + 8.0 * (ax<A, 1>(T) - ax<A, -1>(T))) * G.i12h[A];
-}
-template <int A, class L>
-__device__ __forceinline__ double t_d2(TP<L> T, const Z4cGeo &G) {
-  return (16.0 * (ax<A, -1>(T) + ax<A, 1>(T)) - (ax<A, -2>(T) + ax<A, 2>(T)) - 30.0 * ax<A, 0>(T)) * G.i12hh[A];
-}
-// mixed derivative d_A d_B (A < B): tensor product of 4th-order first differences
-template <int A, int B, int OA, class L>
-__device__ __forceinline__ double t_row(TP<L> T) {
-  constexpr int X0 = (A == 0 ? OA : 0), Y0 = (A == 1 ? OA : 0), Z0 = (A == 2 ? OA : 0);
-  constexpr int BX = (B == 0), BY = (B == 1), BZ = (B == 2);
-  return (at<X0 - 2 * BX, Y0 - 2 * BY, Z0 - 2 * BZ>(T) - at<X0 + 2 * BX, Y0 + 2 * BY, Z0 + 2 * BZ>(T)) +
-         8.0 * (at<X0 + BX, Y0 + BY, Z0 + BZ>(T) - at<X0 - BX, Y0 - BY, Z0 - BZ>(T));
-}
-template <int A, int B, class L>
-__device__ __forceinline__ double t_dd(TP<L> T, const Z4cGeo &G) {
-  return ((t_row<A, B, -2>(T) - t_row<A, B, 2>(T)) + 8.0 * (t_row<A, B, 1>(T) - t_row<A, B, -1>(T))) *
-         G.i144hh[A + B - 1];
-}
-// lop-sided advection: pw = max(beta/h,0)/12, mw = min(beta/h,0)/12 per direction
-template <int A, class L>
-__device__ __forceinline__ double t_adv1(TP<L> T, double pw, double mw) {
-  return pw * ((18.0 * ax<A, 1>(T) - 3.0 * ax<A, -1>(T)) + (ax<A, 3>(T) - 6.0 * ax<A, 2>(T)) -
-               10.0 * ax<A, 0>(T)) +
-         mw * ((6.0 * ax<A, -2>(T) - ax<A, -3>(T)) + (3.0 * ax<A, 1>(T) - 18.0 * ax<A, -1>(T)) +
-               10.0 * ax<A, 0>(T));
-}
-template <class L>
-__device__ __forceinline__ double t_adv(TP<L> T, const double pw[3], const double mw[3]) {
-  return t_adv1<0>(T, pw[0], mw[0]) + t_adv1<1>(T, pw[1], mw[1]) + t_adv1<2>(T, pw[2], mw[2]);
-}
-template <int A, class L>
-__device__ __forceinline__ double t_ko1(TP<L> T) {
-  return (ax<A, -2>(T) + ax<A, 2>(T)) - 4.0 * (ax<A, -1>(T) + ax<A, 1>(T)) + 6.0 * ax<A, 0>(T);
-}
-template <class L>
-__device__ __forceinline__ double t_ko(TP<L> T, const Z4cGeo &G) {
-  return -(t_ko1<0>(T) * G.ih[0] + t_ko1<1>(T) * G.ih[1] + t_ko1<2>(T) * G.ih[2]);
-}
-// all six second derivatives (xx xy xz yy yz zz)
-template <class L>
-__device__ __forceinline__ void t_hess(TP<L> T, const Z4cGeo &G, double d[6]) {
-  d[0] = t_d2<0>(T, G);
-  d[1] = t_dd<0, 1>(T, G);
-  d[2] = t_dd<0, 2>(T, G);
-  d[3] = t_d2<1>(T, G);
-  d[4] = t_dd<1, 2>(T, G);
-  d[5] = t_d2<2>(T, G);
-}
-
-// ---- stencils of the box-edge shell (bam_amr_loops_box.h:186-215,
-// bam_amr_advection.h:90-146): a point one away from an edge uses order-2
-// centred differences and order-2 advection rows, dissipation needs two or
-// more points to every edge, and the advection row shifts away from an edge
-// closer than rstencil.  The shell instantiation (SH = true) of the tile
-// kernel selects these per point.  Every stencil entry with a nonzero
-// coefficient lies inside the box, hence inside the tile's 3-point halo.
-// The advection weights, first-derivative and dissipation coefficients are
-// set once per point, so every point reads the same neighbours at fixed LDS
-// offsets; a neighbour outside the box is read with coefficient 0 from a
-// staging slot that holds box data.  Only the second derivatives branch on
-// the point's order.
-struct Sten {
-  int o2;               // order-2 stencils (one point from an edge)
-  int ko;               // dissipation on (two or more points from every edge)
-  int offp[3], offm[3]; // advection row for beta > 0 / beta < 0 per direction
-  // advection weights of the point's rows, as the reference forms them
-  // (W = -sign(w) w stencil[offset][k] at offset sign(w) (k - offset),
-  // bam_amr_advection.h:90-146): aw[a][o + 3] at offset o = -3..3 along a
-  // (the centre entries unused), awc the sum of the three centre weights
-  double aw[3][7];
-  double awc;
-  // first derivative along a: c1[a] (f(+1) - f(-1)) + c2[a] (f(-2) - f(+2)),
-  // 1/(2h), 0 at order 2 and 8/(12h), 1/(12h) at order 4; kof: 1 where
-  // dissipation is on, else 0
-  double c1[3], c2[3];
-  double kof;
-};
-
-// The point's advection weights along A (w = beta^A / h_A), set once per
-// thread: the stages then read the 19 neighbours at fixed LDS offsets.
-template <int A>
-__device__ __forceinline__ void adv_weights(Sten &S, double w) {
-  const int sg = w > 0.0 ? 1 : -1;
-  const int off = w > 0.0 ? S.offp[A] : S.offm[A];
-#pragma unroll
-  for (int o = -3; o <= 3; o++) {
-    const int k = off + sg * o;  // row entry k lands on offset sg (k - off) = o
-    double c = 0.0;
-    if (S.o2) {
-      if (k >= 0 && k < 3) c = kAdvSt2[off][k];
-    } else {
-      if (k >= 0 && k < 5) c = kAdvSt4[off][k];
-    }
-    S.aw[A][o + 3] = (w == 0.0) ? 0.0 : -sg * w * c;
-  }
-}
-
-template <bool SH, int A, class L>
-__device__ __forceinline__ double s_d1(TP<L> T, const Z4cGeo &G, const Sten &S) {
-  if constexpr (SH) return S.c2[A] * (ax<A, -2>(T) - ax<A, 2>(T)) + S.c1[A] * (ax<A, 1>(T) - ax<A, -1>(T));
-  return t_d1<A>(T, G);
-}
-template <bool SH, class L>
-__device__ __forceinline__ void s_grad(TP<L> T, const Z4cGeo &G, const Sten &S, double d[3]) {
-  d[0] = s_d1<SH, 0>(T, G, S);
-  d[1] = s_d1<SH, 1>(T, G, S);
-  d[2] = s_d1<SH, 2>(T, G, S);
-}
-template <int A, int B, class L>
-__device__ __forceinline__ double t_dd2(TP<L> T, const Z4cGeo &G) {
-  constexpr int AX = (A == 0), AY = (A == 1), AZ = (A == 2), BX = (B == 0), BY = (B == 1), BZ = (B == 2);
-  return ((at<AX + BX, AY + BY, AZ + BZ>(T) - at<AX - BX, AY - BY, AZ - BZ>(T)) -
-          (at<-AX + BX, -AY + BY, -AZ + BZ>(T) - at<-AX - BX, -AY - BY, -AZ - BZ>(T))) *
-         G.i4hh[A + B - 1];
-}
-template <bool SH, class L>
-__device__ __forceinline__ void s_hess(TP<L> T, const Z4cGeo &G, const Sten &S, double d[6]) {
-  if (SH && S.o2) {
-    d[0] = (ax<0, -1>(T) + ax<0, 1>(T) - 2.0 * ax<0, 0>(T)) * G.ihh[0];
-    d[1] = t_dd2<0, 1>(T, G);
-    d[2] = t_dd2<0, 2>(T, G);
-    d[3] = (ax<1, -1>(T) + ax<1, 1>(T) - 2.0 * ax<1, 0>(T)) * G.ihh[1];
-    d[4] = t_dd2<1, 2>(T, G);
-    d[5] = (ax<2, -1>(T) + ax<2, 1>(T) - 2.0 * ax<2, 0>(T)) * G.ihh[2];
-    return;
-  }
-  t_hess(T, G, d);
-}
-// advection with the point's weights (shell) or the lop-sided rows (bulk)
-template <int A, class L>
-__device__ __forceinline__ double s_advw1(TP<L> T, const double w[7]) {
-  return w[0] * ax<A, -3>(T) + w[1] * ax<A, -2>(T) + w[2] * ax<A, -1>(T) + w[4] * ax<A, 1>(T) +
-         w[5] * ax<A, 2>(T) + w[6] * ax<A, 3>(T);
-}
-template <bool SH, class L>
-__device__ __forceinline__ double s_adv(TP<L> T, const double pw[3], const double mw[3], const Sten &S) {
-  if constexpr (SH)
-    return S.awc * at<0, 0, 0>(T) + s_advw1<0>(T, S.aw[0]) + s_advw1<1>(T, S.aw[1]) + s_advw1<2>(T, S.aw[2]);
-  return t_adv(T, pw, mw);
-}
-template <bool SH, class L>
-__device__ __forceinline__ double s_ko(TP<L> T, const Z4cGeo &G, const Sten &S) {
-  if constexpr (SH) return S.kof * t_ko(T, G);
-  return t_ko(T, G);
-}
-
-// Staging of one field into the LDS tile, software-pipelined: the global
-// loads of the next field are issued into registers (NLOAD per thread, all
-// in flight together) before the current field is computed, and written to
-// LDS between two barriers at the start of the next stage.
-// staging order of the 25 fields: gt_ij, Gamma^i, chi, alpha, Khat, Theta,
-// At_ij, beta^i, B^i
-__device__ constexpr int STAGE_ORDER[25] = {0,  1,  2,  3,  4,  5,  14, 15, 16, 6,  18, 13, 17,
-                                            7,  8,  9,  10, 11, 12, 19, 20, 21, 22, 23, 24};
-
-template <class L>
-struct Stager {
-  static constexpr int NLOAD = L::NLOAD;
-  int goff[NLOAD];
-  unsigned ok;      // bit k: slot k lies inside the tile and the box
-  long cbase;       // linear index of the tile corner (i0-3, j0-3, k0-3); may lie before the box
-  double pf[NLOAD];
-  __device__ Stager(const Z4cGeo &G, int i0, int j0, int k0, int tid) {
-    cbase = G.noffset + (i0 - HALO) + G.sj * (j0 - HALO) + G.sk * (k0 - HALO);
-    ok = 0;
-#pragma unroll
-    for (int k = 0; k < NLOAD; k++) {
-      const int idx = tid + k * NTHR;
-      const int x = idx % L::SX, y = (idx / L::SX) % L::SY, z = idx / (L::SX * L::SY);
-      const int gi = i0 - HALO + x, gj = j0 - HALO + y, gk = k0 - HALO + z;
-      const bool in = idx < L::TILE && x < L::WX && gi >= 0 && gj >= 0 && gk >= 0 && gi < G.m && gj < G.n && gk < G.o;
-      goff[k] = in ? (int)(x + G.sj * y + G.sk * z) : 0;
-      ok |= in ? (1u << k) : 0u;
-    }
-  }
-  // slots outside the box are staged as 0; no stencil of a computed point reads them
-  __device__ __forceinline__ void load(const double *__restrict__ f) {
-#pragma unroll
-    for (int k = 0; k < NLOAD; k++) pf[k] = (ok >> k & 1u) ? f[cbase + goff[k]] : 0.0;
-  }
-  __device__ __forceinline__ void commit(double *tile, int tid) {
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < NLOAD; k++)
-      if (tid + k * NTHR < L::TILE) tile[tid + k * NTHR] = pf[k];
-    __syncthreads();
-  }
-};
-
-// Staging through the LDS-DMA path: global_load_lds moves each field
-// straight from HBM into one of NB LDS buffers (no registers, no ds_write), so
-// NB - 1 fields are in flight while one is computed.  A wave's 64 lanes write
-// 64 consecutive units of LDS (lane l -> unit l), so the tile is cut into
-// chunks of 64 units, NPER per wave.  VEC = 1: a unit is one dword, the low
-// (even unit) or high half of a tile element; VEC = 4: a unit is 16 bytes,
-// the two tile elements (x, x + 1) with x even, which needs an even row
-// length and 16-byte aligned pairs in HBM (checked by the host).  Slots of
-// the tile outside the box load the nearest point of the box (a pair stays a
-// pair), so that every staged value is box data: the shell's advection reads
-// such slots with weight 0.
-#define BH_LDS(p) ((__attribute__((address_space(3))) void *)(p))
-template <class L, int NB, int VEC>
-struct DmaStager {
-  static_assert(VEC == 1 || VEC == 4, "dword or 16-byte units");
-  static_assert(VEC == 1 || (L::SX % 2 == 0 && L::TX % 2 == 0), "16-byte units need even rows and tile steps");
-  static constexpr int NW = NTHR / 64;
-  static constexpr int NUNIT = VEC == 1 ? 2 * L::TILE : L::TILE / 2;
-  static constexpr int NCH = (NUNIT + 63) / 64;
-  static constexpr int NPER = (NCH + NW - 1) / NW;
-  static constexpr int CHD = 64 * VEC / 2;      // doubles per chunk
-  static constexpr int BUFD = NPER * NW * CHD;  // doubles per buffer, padded to whole chunks
-  static_assert(NB >= 2 && (NB - 2) * NPER <= 63, "vmcnt range");
-  unsigned boff[NPER];  // byte offset of each chunk's unit from the field's base
-  int wave;
-  __device__ DmaStager(const Z4cGeo &G, int i0, int j0, int k0, int tid) {
-    const int lane = tid & 63;
-    wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-#pragma unroll
-    for (int c = 0; c < NPER; c++) {
-      const int d = (wave * NPER + c) * 64 + lane;
-      const int e = VEC == 1 ? d >> 1 : 2 * d;
-      const int x = e % L::SX, y = (e / L::SX) % L::SY, z = e / (L::SX * L::SY);
-      const int gi = i0 - HALO + x, gj = j0 - HALO + y, gk = k0 - HALO + z;
-      const bool in = e < L::TILE && x < L::WX;
-      // clamped into the box; for 16-byte units gi is even and so is the
-      // box's row length, so the clamped pair is (0, 1) or (m - 2, m - 1)
-      const int ci = min(max(gi, 0), G.m - (VEC == 1 ? 1 : 2)), cj = min(max(gj, 0), G.n - 1),
-                ck = min(max(gk, 0), G.o - 1);
-      const long el = in ? G.noffset + ci + G.sj * cj + G.sk * ck : G.noffset;
-      boff[c] = (unsigned)(el * 8 + (VEC == 1 && in ? (d & 1) * 4 : 0));
-    }
-  }
-  __device__ __forceinline__ void issue(const double *f, double *buf) const {
-#pragma unroll
-    for (int c = 0; c < NPER; c++) {
-      const void *src = (const void *)((const char *)f + boff[c]);
-      if constexpr (VEC == 1)
-        __builtin_amdgcn_global_load_lds(src, BH_LDS(buf + (wave * NPER + c) * CHD), 4, 0, 0);
-      else
-        __builtin_amdgcn_global_load_lds(src, BH_LDS(buf + (wave * NPER + c) * CHD), 16, 0, 0);
-    }
-  }
-};
-// s_waitcnt vmcnt(n) lgkmcnt(0) (expcnt not waited), n a small constant
-template <int N>
-__device__ __forceinline__ void wait_vm_lgkm0() {
-  static_assert(N >= 0 && N <= 63, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));
-}
-template <int NPER>
-__device__ __forceinline__ void wait_fields_after(int k) {
-  switch (k) {
-    case 0: wait_vm_lgkm0<0>(); break;
-    case 1: wait_vm_lgkm0<NPER>(); break;
-    case 2: wait_vm_lgkm0<(2 * NPER <= 63 ? 2 * NPER : 0)>(); break;
-    default: wait_vm_lgkm0<(3 * NPER <= 63 ? 3 * NPER : 0)>(); break;
-  }
-}
-// workgroup barrier without a memory fence (a fence would also wait for the
-// LDS-DMA loads still in flight); the empty asm statements keep the compiler
-// from moving memory accesses across it
-__device__ __forceinline__ void bare_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// Pin a value in registers at this point of the program: an empty volatile
-// asm that reads and writes it.  Placed after each staged field, it keeps the
-// compiler from sinking that field's arithmetic past the next stage's
-// barrier, which would keep every staged tile's values live to the end of
-// the kernel (and spill).
-__device__ __forceinline__ void pin(double &x) { asm volatile("" : "+v"(x)); }
-template <int N>
-__device__ __forceinline__ void pin(double (&a)[N]) {
-#pragma unroll
-  for (int i = 0; i < N; i++) pin(a[i]);
-}
-
-// Regions of one launch: index ranges [lo, hi] of boxes of a level (bulk
-// regions, or slabs of the box-edge shell), each with its box geometry, and
-// the first block of each region.  All boxes of a level are computed by one
-// launch per tile layout.
-// The grid spacing constants are common to the regions of one launch (one
-// level), so a region carries only integer geometry.
-constexpr int kMaxRegions = 32;
-struct RegionGeo {
-  int m, n, o;
-  int lo[3], hi[3];
-  long noffset, sj, sk;
-};
-struct Spacing {
-  double h[3], ih[3], i12h[3], i12hh[3], i144hh[3], i2h[3], ihh[3], i4hh[3];
-};
-struct TileJobs {
-  int n;
-  int blk0[kMaxRegions + 1];  // first tile of each region; blk0[n] = number of tiles
-  int xcd;                    // 1: XCD-aware numbering of the tiles (grid padded to a multiple of 8)
-  RegionGeo reg[kMaxRegions];
-  Spacing sp;
-};
-static_assert(sizeof(TileJobs) <= 3072, "kernel argument size");
-static_assert(sizeof(Z4cPtrs) + sizeof(TileJobs) + sizeof(Z4cK) + sizeof(int *) <= 4096,
-              "arguments of the tile kernel within 4 KiB");
-
-// SH = false: every point of the regions is >= 3 from each edge (standard
-// stencils).  SH = true: the regions are slabs of the box-edge shell; only
-// points closer than 3 to an edge are computed, with the per-point rules of
-// Sten.
-template <class L, int NB, int VEC>
-struct StageBuf {  // LDS doubles of the staging buffers
-  static constexpr int n = NB * DmaStager<L, NB, VEC>::BUFD;
-};
-template <class L, int VEC>
-struct StageBuf<L, 0, VEC> {
-  static constexpr int n = L::TILE;
-};
-
-// NB = 0: one LDS tile, staged through registers (Stager); NB >= 2: NB LDS
-// buffers filled by the LDS-DMA path (DmaStager).  OCC: blocks per CU the
-// register allocation must allow (2 caps a thread at 256 registers, with
-// spills, for two waves per SIMD).
-template <class L, bool SH, int NB, int VEC, int OCC>
-__global__ void __launch_bounds__(NTHR, OCC) z4c_rhs_tile(Z4cPtrs P, TileJobs J, Z4cK K, int *flag) {
-  __shared__ double tile[StageBuf<L, NB, VEC>::n];
-  // Tile of this block.  Workgroups are dispatched to the 8 XCDs round-robin
-  // (workgroup w to XCD w mod 8), each XCD with its own L2.  With xcd set,
-  // workgroup w takes tile (w mod 8) * per + w / 8, so every XCD works through
-  // one contiguous range of tiles and neighbouring tiles, which stage the same
-  // halo points, meet in the same L2.
-  int t = (int)blockIdx.x;
-  if (J.xcd) {
-    const int per = (int)gridDim.x / 8;
-    t = (t % 8) * per + t / 8;
-    if (t >= J.blk0[J.n]) return;  // padding workgroup (whole block, before any barrier)
-  }
-  // region of this block (uniform): the regions' tiles are numbered in order
-  int r = 0;
-  while (r + 1 < J.n && t >= J.blk0[r + 1]) r++;
-  // copies: indexing the argument array by r through a reference would stage it in scratch
-  const RegionGeo Rg = J.reg[r];
-  Z4cGeo G;
-  G.m = Rg.m;
-  G.n = Rg.n;
-  G.o = Rg.o;
-  G.noffset = Rg.noffset;
-  G.sj = Rg.sj;
-  G.sk = Rg.sk;
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    G.lo[a] = Rg.lo[a];
-    G.hi[a] = Rg.hi[a];
-    G.h[a] = J.sp.h[a];
-    G.ih[a] = J.sp.ih[a];
-    G.i12h[a] = J.sp.i12h[a];
-    G.i12hh[a] = J.sp.i12hh[a];
-    G.i144hh[a] = J.sp.i144hh[a];
-    G.i2h[a] = J.sp.i2h[a];
-    G.ihh[a] = J.sp.ihh[a];
-    G.i4hh[a] = J.sp.i4hh[a];
-  }
-  G.edge_only = 0;
-  const int b = t - J.blk0[r];
-  const int ntx = (G.hi[0] - G.lo[0] + L::TX) / L::TX, nty = (G.hi[1] - G.lo[1] + L::TY) / L::TY;
-  const int tid = (int)threadIdx.x;
-  int tx, ty, tz;
-  L::coords(tid, tx, ty, tz);
-  const int i0 = G.lo[0] + (b % ntx) * L::TX, j0 = G.lo[1] + ((b / ntx) % nty) * L::TY,
-            k0 = G.lo[2] + (b / (ntx * nty)) * L::TZ;
-  const int i = i0 + tx, j = j0 + ty, k = k0 + tz;
-  Sten S{};
-  bool active = (i <= G.hi[0] && j <= G.hi[1] && k <= G.hi[2]);
-  if (SH) {
-    // positions past hi (padding threads, never stored) are clamped to hi, so
-    // that their rows and stencil reach stay within the tables and the halo
-    const int pos[3] = {min(i, G.hi[0]), min(j, G.hi[1]), min(k, G.hi[2])};
-    const int pmax[3] = {G.m - 1, G.n - 1, G.o - 1};
-    int dmin = 1 << 30;
-#pragma unroll
-    for (int a = 0; a < 3; a++) dmin = min(dmin, min(pos[a], pmax[a] - pos[a]));
-    active = active && dmin <= 2;
-    S.o2 = dmin == 1;
-    S.ko = dmin >= 2;
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      const int dl = pos[a], dh = pmax[a] - pos[a];
-      if (S.o2) {
-        S.offm[a] = dl >= 2 ? 0 : 2 - dl;
-        S.offp[a] = dh >= 2 ? 0 : 2 - dh;
-      } else {
-        S.offm[a] = (dl >= 3 ? 0 : 3 - dl) + 1;
-        S.offp[a] = (dh >= 3 ? 0 : 3 - dh) + 1;
-      }
-    }
-  }
-  const long q = G.noffset + i + G.sj * j + G.sk * k;
-  const int toff = tx + L::SX * (ty + L::SY * tz);
-  TP<L> T{tile + toff};
-  const double *const *u = P.u;
-
-  // the first fields' transfers go out before the point values are loaded,
-  // so that a block waits for one round trip to HBM at its start, not two
-  using St = typename std::conditional<NB == 0, Stager<L>, DmaStager<L, (NB == 0 ? 2 : NB), VEC>>::type;
-  St st(G, i0, j0, k0, tid);
-  constexpr int NBUF = NB == 0 ? 1 : NB;
-  constexpr int BUFD = StageBuf<L, NB, VEC>::n / NBUF;
-  if constexpr (NB == 0) {
-    st.load(u[STAGE_ORDER[0]]);
-  } else {
-#pragma unroll
-    for (int p = 0; p < NB - 1; p++) st.issue(u[STAGE_ORDER[p]], tile + p * BUFD);
-  }
-
-  // point values; threads outside the box use flat data so that their
-  // (discarded) arithmetic stays finite
-  double g[6], A[6], Gm[3], beta[3], Bv[3];
-  double chi = 1.0, Khat = 0.0, Theta = 0.0, alpha = 1.0;
-  for (int c = 0; c < 6; c++) {
-    g[c] = (c == 0 || c == 3 || c == 5) ? 1.0 : 0.0;
-    A[c] = 0.0;
-  }
-  for (int a = 0; a < 3; a++) Gm[a] = beta[a] = Bv[a] = 0.0;
-  if (active) {
-#pragma unroll
-    for (int c = 0; c < 6; c++) {
-      g[c] = u[c][q];
-      A[c] = u[7 + c][q];
-    }
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      Gm[a] = u[14 + a][q];
-      beta[a] = u[19 + a][q];
-      Bv[a] = u[22 + a][q];
-    }
-    chi = u[6][q];
-    Khat = u[13][q];
-    Theta = u[17][q];
-    alpha = u[18][q];
-  }
-  // stage s: make field s visible in LDS, start the transfer of a later field
-  auto advance = [&](int sidx) {
-    if constexpr (NB == 0) {
-      st.commit(tile, tid);
-      if (sidx + 1 < 25) st.load(u[STAGE_ORDER[sidx + 1]]);
-    } else {
-      // this wave's loads of field sidx are done once no more than the later
-      // fields' loads are outstanding; the barrier makes every wave's done
-      wait_fields_after<St::NPER>(min(NB - 2, 24 - sidx));
-      bare_barrier();
-      // the buffer of field sidx + NB - 1 held field sidx - 1, whose reads
-      // every wave completed before the barrier
-      if (sidx + NB - 1 < 25) st.issue(u[STAGE_ORDER[sidx + NB - 1]], tile + ((sidx + NB - 1) % NB) * BUFD);
-      T.p = tile + (sidx % NB) * BUFD + toff;
-    }
-  };
-  double pw[3], mw[3];
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    const double w = beta[a] * G.ih[a];
-    pw[a] = (w > 0.0 ? w : 0.0) * (1.0 / 12.0);
-    mw[a] = (w < 0.0 ? w : 0.0) * (1.0 / 12.0);
-  }
-  if constexpr (SH) {
-    adv_weights<0>(S, beta[0] * G.ih[0]);
-    adv_weights<1>(S, beta[1] * G.ih[1]);
-    adv_weights<2>(S, beta[2] * G.ih[2]);
-    S.awc = S.aw[0][3] + S.aw[1][3] + S.aw[2][3];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      S.c1[a] = S.o2 ? G.i2h[a] : 8.0 * G.i12h[a];
-      S.c2[a] = S.o2 ? 0.0 : G.i12h[a];
-    }
-    S.kof = S.ko ? 1.0 : 0.0;
-  }
-  const bool ko = (K.order_dissipation == 4);
-  const double eps = ko ? K.dissfactor : 0.0;
-
-  // inverse conformal metric
-  double ig[6];
-  ig[0] = g[3] * g[5] - g[4] * g[4];
-  ig[1] = g[2] * g[4] - g[1] * g[5];
-  ig[2] = g[1] * g[4] - g[2] * g[3];
-  ig[3] = g[0] * g[5] - g[2] * g[2];
-  ig[4] = g[1] * g[2] - g[0] * g[4];
-  ig[5] = g[0] * g[3] - g[1] * g[1];
-  const double detginv = 1.0 / (g[0] * ig[0] + g[1] * ig[1] + g[2] * ig[2]);
-#pragma unroll
-  for (int c = 0; c < 6; c++) ig[c] *= detginv;
-  auto trace = [&](const double *t6) {
-    return ig[0] * t6[0] + ig[3] * t6[3] + ig[5] * t6[5] + 2.0 * (ig[1] * t6[1] + ig[2] * t6[2] + ig[4] * t6[4]);
-  };
-  auto contract = [&](const double *x, const double *y) {
-    return ig[0] * x[0] * y[0] + ig[3] * x[1] * y[1] + ig[5] * x[2] * y[2] + ig[1] * (x[0] * y[1] + x[1] * y[0]) +
-           ig[2] * (x[0] * y[2] + x[2] * y[0]) + ig[4] * (x[1] * y[2] + x[2] * y[1]);
-  };
-
-  double rhs[25];
-  double R[6];  // Ricci accumulators (conformal + phi part)
-
-  // ---- conformal metric: first derivatives, Laplacian part of Ricci
-  double dg[3][6];
-static_for<6>([&](auto I_) {
-    constexpr int ab = decltype(I_)::value;
-    advance(ab);
-    dg[0][ab] = s_d1<SH, 0>(T, G, S);
-    dg[1][ab] = s_d1<SH, 1>(T, G, S);
-    dg[2][ab] = s_d1<SH, 2>(T, G, S);
-    double h6[6];
-    s_hess<SH>(T, G, S, h6);
-    R[ab] = -0.5 * trace(h6);
-    rhs[ab] = s_adv<SH>(T, pw, mw, S) + eps * s_ko<SH>(T, G, S);
-    pin(dg[0][ab]);
-    pin(dg[1][ab]);
-    pin(dg[2][ab]);
-    pin(R[ab]);
-    pin(rhs[ab]);
-  });
-  // Christoffels
-  double Gu[3][6], Gfg[3];
-  {
-    double Gd[3][6];
-#pragma unroll
-    for (int c = 0; c < 3; c++)
-#pragma unroll
-      for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int b = a; b < 3; b++)
-          Gd[c][sy(a, b)] = 0.5 * (dg[a][sy(b, c)] + dg[b][sy(a, c)] - dg[c][sy(a, b)]);
-#pragma unroll
-    for (int c = 0; c < 3; c++)
-#pragma unroll
-      for (int ab = 0; ab < 6; ab++)
-        Gu[c][ab] = ig[sy(c, 0)] * Gd[0][ab] + ig[sy(c, 1)] * Gd[1][ab] + ig[sy(c, 2)] * Gd[2][ab];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-      Gfg[a] = ig[0] * Gu[a][0] + ig[3] * Gu[a][3] + ig[5] * Gu[a][5] +
-               2.0 * (ig[1] * Gu[a][1] + ig[2] * Gu[a][2] + ig[4] * Gu[a][4]);
-    // quadratic Christoffel terms of R_ab
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = a; b < 3; b++) {
-        double s = 0.0;
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-#pragma unroll
-          for (int d = 0; d < 3; d++) {
-            double t = 0.0;
-#pragma unroll
-            for (int e = 0; e < 3; e++)
-              t += Gu[e][sy(c, a)] * Gd[b][sy(e, d)] + Gu[e][sy(c, b)] * Gd[a][sy(e, d)] +
-                   Gu[e][sy(a, d)] * Gd[e][sy(c, b)];
-            s += ig[sy(c, d)] * t;
-          }
-        double t2 = 0.0;
-#pragma unroll
-        for (int c = 0; c < 3; c++) t2 += Gfg[c] * (Gd[a][sy(b, c)] + Gd[b][sy(a, c)]);
-        R[sy(a, b)] += s + 0.5 * t2;
-      }
-  }
-  pin(R);
-  pin(Gu[0]);
-  pin(Gu[1]);
-  pin(Gu[2]);
-  pin(Gfg);
-
-  // ---- Gamma^i: + 1/2 (g_ca d_b G^c + g_cb d_a G^c) in R_ab
-  double advG[3], koG[3];
-static_for<3>([&](auto I_) {
-    constexpr int c = decltype(I_)::value;
-    advance(6 + c);
-    double dG[3];
-    s_grad<SH>(T, G, S,dG);
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = a; b < 3; b++) R[sy(a, b)] += 0.5 * (g[sy(c, a)] * dG[b] + g[sy(c, b)] * dG[a]);
-    advG[c] = s_adv<SH>(T, pw, mw, S);
-    koG[c] = eps * s_ko<SH>(T, G, S);
-    pin(R);
-    pin(advG[c]);
-    pin(koG[c]);
-  });
-
-  // ---- conformal factor
-  const double chig = (chi < K.chiDivFloor) ? K.chiDivFloor : chi;
-  const double oocp = 1.0 / K.chipsipower;
-  const double psim4 = exp(-4.0 * oocp * log(chig));
-  const double oochig = 1.0 / chig;
-  double dchi[3], df[3];
-  {
-    advance(9);
-    s_grad<SH>(T, G, S,dchi);
-    double h6[6];
-    s_hess<SH>(T, G, S, h6);
-    rhs[6] = s_adv<SH>(T, pw, mw, S) + eps * s_ko<SH>(T, G, S);
-#pragma unroll
-    for (int a = 0; a < 3; a++) df[a] = oocp * dchi[a] * oochig;
-    double cddf[6];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = a; b < 3; b++) {
-        const int ab = sy(a, b);
-        cddf[ab] = oocp * h6[ab] * oochig - K.chipsipower * df[a] * df[b] -
-                   (Gu[0][ab] * df[0] + Gu[1][ab] * df[1] + Gu[2][ab] * df[2]);
-      }
-    const double trcddf = trace(cddf);
-    const double dfdf = contract(df, df);
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = a; b < 3; b++) {
-        const int ab = sy(a, b);
-        R[ab] += 4.0 * df[a] * df[b] - 2.0 * cddf[ab] - 2.0 * g[ab] * trcddf - 4.0 * g[ab] * dfdf;
-      }
-    pin(R);
-    pin(dchi);
-    pin(df);
-    pin(rhs[6]);
-  }
-
-  // ---- lapse
-  double da[3], cdda[6];
-  {
-    advance(10);
-    s_grad<SH>(T, G, S,da);
-    double h6[6];
-    s_hess<SH>(T, G, S, h6);
-    rhs[18] = K.oplogwithshift * s_adv<SH>(T, pw, mw, S) + eps * s_ko<SH>(T, G, S);
-    const double dfda = contract(df, da);
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = a; b < 3; b++) {
-        const int ab = sy(a, b);
-        cdda[ab] = h6[ab] - (Gu[0][ab] * da[0] + Gu[1][ab] * da[1] + Gu[2][ab] * da[2]) -
-                   2.0 * (df[a] * da[b] + df[b] * da[a] - g[ab] * dfda);
-      }
-    pin(da);
-    pin(cdda);
-    pin(rhs[18]);
-  }
-  const double trcdda = psim4 * trace(cdda);
-
-  // ---- Khat and Theta: 2 dKhat + dTheta
-  double dKT[3], koT;
-  {
-    advance(11);
-    dKT[0] = 2.0 * s_d1<SH, 0>(T, G, S);
-    dKT[1] = 2.0 * s_d1<SH, 1>(T, G, S);
-    dKT[2] = 2.0 * s_d1<SH, 2>(T, G, S);
-    rhs[13] = s_adv<SH>(T, pw, mw, S) + eps * s_ko<SH>(T, G, S);
-    pin(dKT);
-    pin(rhs[13]);
-    advance(12);
-    dKT[0] += s_d1<SH, 0>(T, G, S);
-    dKT[1] += s_d1<SH, 1>(T, G, S);
-    dKT[2] += s_d1<SH, 2>(T, G, S);
-    rhs[17] = s_adv<SH>(T, pw, mw, S);  // KO of Theta is added after the zeroThetaRHS factor
-    koT = eps * s_ko<SH>(T, G, S);
-    pin(dKT);
-    pin(rhs[17]);
-    pin(koT);
-  }
-
-  // ---- trace-free extrinsic curvature: advection and dissipation only
-static_for<6>([&](auto I_) {
-    constexpr int ab = decltype(I_)::value;
-    advance(13 + ab);
-    rhs[7 + ab] = s_adv<SH>(T, pw, mw, S) + eps * s_ko<SH>(T, G, S);
-    pin(rhs[7 + ab]);
-  });
-
-  // ---- shift: d_a beta^b, g^bc d_b d_c beta^a, (1/3) d_a d_c beta^c
-  double db[3][3], pG[3], ootd[3];
-static_for<3>([&](auto I_) {
-    constexpr int c = decltype(I_)::value;
-    advance(19 + c);
-    db[0][c] = s_d1<SH, 0>(T, G, S);
-    db[1][c] = s_d1<SH, 1>(T, G, S);
-    db[2][c] = s_d1<SH, 2>(T, G, S);
-    double h6[6];
-    s_hess<SH>(T, G, S, h6);
-    pG[c] = trace(h6);
-#pragma unroll
-    for (int a = 0; a < 3; a++) ootd[a] = (c == 0 ? 0.0 : ootd[a]) + (1.0 / 3.0) * h6[sy(a, c)];
-    rhs[19 + c] = K.withShiftadv * s_adv<SH>(T, pw, mw, S) + eps * s_ko<SH>(T, G, S);
-    pin(db[0][c]);
-    pin(db[1][c]);
-    pin(db[2][c]);
-    pin(pG[c]);
-    pin(ootd);
-    pin(rhs[19 + c]);
-  });
-  // ---- B: advection and dissipation only
-static_for<3>([&](auto I_) {
-    constexpr int c = decltype(I_)::value;
-    advance(22 + c);
-    rhs[22 + c] = (K.withB != 0.0 ? K.withBadv * s_adv<SH>(T, pw, mw, S) : 0.0) + eps * s_ko<SH>(T, G, S);
-    pin(rhs[22 + c]);
-  });
-
-  // ---- algebra
-  double Ainv[6], AA[6];
-  {
-    double Au[3][3];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = 0; b < 3; b++)
-        Au[a][b] = ig[sy(a, 0)] * A[sy(0, b)] + ig[sy(a, 1)] * A[sy(1, b)] + ig[sy(a, 2)] * A[sy(2, b)];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = a; b < 3; b++) {
-        Ainv[sy(a, b)] = Au[a][0] * ig[sy(0, b)] + Au[a][1] * ig[sy(1, b)] + Au[a][2] * ig[sy(2, b)];
-        AA[sy(a, b)] = A[sy(a, 0)] * Au[0][b] + A[sy(a, 1)] * Au[1][b] + A[sy(a, 2)] * Au[2][b];
-      }
-  }
-  const double cAA = trace(AA);
-  const double K_ = Khat + 2.0 * Theta;
-  double divAinv[3];
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    double s = 0.0;
-#pragma unroll
-    for (int bc = 0; bc < 6; bc++) s += ((bc == 0 || bc == 3 || bc == 5) ? 1.0 : 2.0) * Gu[a][bc] * Ainv[bc];
-    s -= 1.5 * oochig * (Ainv[sy(a, 0)] * dchi[0] + Ainv[sy(a, 1)] * dchi[1] + Ainv[sy(a, 2)] * dchi[2]);
-    s -= (1.0 / 3.0) * (ig[sy(a, 0)] * dKT[0] + ig[sy(a, 1)] * dKT[1] + ig[sy(a, 2)] * dKT[2]);
-    divAinv[a] = s;
-  }
-  const double Rhat = psim4 * trace(R);
-  const double Hhat = Rhat + 2.0 * K_ * K_ / 3.0 - cAA;
-  const double divbeta = db[0][0] + db[1][1] + db[2][2];
-  const double tdb = (2.0 / 3.0) * divbeta;
-
-#pragma unroll
-  for (int a = 0; a < 3; a++)
-#pragma unroll
-    for (int b = a; b < 3; b++) {
-      const int ab = sy(a, b);
-      double lg = -g[ab] * tdb, lA = -A[ab] * tdb;
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        lg += db[a][c] * g[sy(b, c)] + db[b][c] * g[sy(a, c)];
-        lA += db[a][c] * A[sy(b, c)] + db[b][c] * A[sy(a, c)];
-      }
-      rhs[ab] += -2.0 * alpha * A[ab] + lg;
-      rhs[7 + ab] += psim4 * (-cdda[ab] + alpha * R[ab]) - (1.0 / 3.0) * g[ab] * (-trcdda + alpha * Rhat) +
-                     alpha * (K_ * A[ab] - 2.0 * AA[ab]) + lA;
-    }
-  double rG[3];
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    const double pseudolie = pG[a] + ig[sy(a, 0)] * ootd[0] + ig[sy(a, 1)] * ootd[1] + ig[sy(a, 2)] * ootd[2] -
-                             (Gfg[0] * db[0][a] + Gfg[1] * db[1][a] + Gfg[2] * db[2][a]) + Gfg[a] * tdb + advG[a];
-    rG[a] = -2.0 * (Ainv[sy(a, 0)] * da[0] + Ainv[sy(a, 1)] * da[1] + Ainv[sy(a, 2)] * da[2]) +
-            2.0 * alpha * divAinv[a] - 2.0 * alpha * K.kappa1 * (Gm[a] - Gfg[a]) + pseudolie;
-    rhs[14 + a] = rG[a] + koG[a];
-  }
-  rhs[13] += -trcdda + alpha * (cAA + K_ * K_ / 3.0) + K.kappa1 * (1.0 - K.kappa2) * alpha * Theta;
-  rhs[6] += (K.chipsipower / 6.0) * chig * (divbeta - alpha * K_);
-  rhs[17] = (alpha * (0.5 * Hhat - (2.0 + K.kappa2) * K.kappa1 * Theta) + rhs[17]) * K.zeroThetaRHS + koT;
-
-  const double falpha =
-      K.oploglapse * K.lapseharmonicf + K.oploglapse2 * (8.0 / 3.0) / (3.0 - alpha) + K.harmoniclapse * alpha;
-  rhs[18] -= falpha * alpha * Khat;
-  if (K.withB != 0.0) {
-    const double betaF = K.shiftgammacoeff * pow(alpha, K.shiftalphapower);
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      rhs[19 + a] += (K.gamma2factor + K.gamma0factor * betaF) * Bv[a];
-      rhs[22 + a] += (K.gamma0factor + K.gamma2factor * betaF) * (rG[a] - K.withGadv * advG[a]) -
-                     K.shiftdriver * Bv[a];
-    }
-  } else {
-#pragma unroll
-    for (int a = 0; a < 3; a++) rhs[19 + a] += Gm[a] - K.shiftdriver * beta[a];
-  }
-  if (!active) return;
-  bool finite = true;
-#pragma unroll
-  for (int v = 0; v < 25; v++) finite = finite && isfinite(rhs[v]);
-  if (!finite) *flag = 1;
-  store_point(P, K, q, rhs);
-}
-
 // ------------------------------------------------------------------ kernels
 // all computed points that are not in [blo, bhi] (the bulk region), or all
 // computed points when edge_only == 0
@@ -1490,6 +556,7 @@ static Z4cK make_k(const bamhip_z4c_params *p, double c) {
   K.shiftdriver = p->shiftdriver;
   K.chiDivFloor = p->chiDivFloor;
   K.chipsipower = p->chipsipower;
+  K.oocp = 1.0 / p->chipsipower;
   K.c = c;
   K.addlinear = (c != 0.0);
   K.rk = 0;
@@ -1534,7 +601,6 @@ static void make_geo(const DevBox &B, Z4cGeo &G) {
 struct LevelTiles {
   std::vector<Z4cGeo> bulk;
   std::vector<Z4cGeo> sx, sy, sz;  // shell as slabs (up to two points thick) normal to x, y, z
-  std::vector<Z4cGeo> lx, ly, lz;  // the same slabs cut into single layers
 };
 
 static void add_region(std::vector<Z4cGeo> &v, const Z4cGeo &G0, const int lo[3], const int hi[3]) {
@@ -1547,64 +613,8 @@ static void add_region(std::vector<Z4cGeo> &v, const Z4cGeo &G0, const int lo[3]
   v.push_back(G);
 }
 
-template <class L>
-static int ntiles(const Z4cGeo &G) {
-  return ((G.hi[0] - G.lo[0] + L::TX) / L::TX) * ((G.hi[1] - G.lo[1] + L::TY) / L::TY) *
-         ((G.hi[2] - G.lo[2] + L::TZ) / L::TZ);
-}
-
-// one launch per kMaxRegions regions of a layout
 static int g_xcd_map = 1;  // XCD-aware tile numbering in the tile kernels
-
-static bool same_spacing(const Z4cGeo &a, const Z4cGeo &b) {
-  return a.h[0] == b.h[0] && a.h[1] == b.h[1] && a.h[2] == b.h[2];
-}
-
-// one launch per kMaxRegions regions of a layout (and per grid spacing)
-template <class L, bool SH, int NB, int VEC, int OCC>
-static int launch_regions(const Z4cPtrs &P, const std::vector<Z4cGeo> &regs, const Z4cK &K, int *flag,
-                          hipStream_t st) {
-  size_t r0 = 0;
-  while (r0 < regs.size()) {
-    TileJobs J{};
-    const Z4cGeo &G0 = regs[r0];
-    for (int a = 0; a < 3; a++) {
-      J.sp.h[a] = G0.h[a];
-      J.sp.ih[a] = G0.ih[a];
-      J.sp.i12h[a] = G0.i12h[a];
-      J.sp.i12hh[a] = G0.i12hh[a];
-      J.sp.i144hh[a] = G0.i144hh[a];
-      J.sp.i2h[a] = G0.i2h[a];
-      J.sp.ihh[a] = G0.ihh[a];
-      J.sp.i4hh[a] = G0.i4hh[a];
-    }
-    int blk = 0;
-    J.n = 0;
-    while (r0 < regs.size() && J.n < kMaxRegions && same_spacing(regs[r0], G0)) {
-      const Z4cGeo &G = regs[r0++];
-      RegionGeo &Rg = J.reg[J.n];
-      Rg.m = G.m;
-      Rg.n = G.n;
-      Rg.o = G.o;
-      Rg.noffset = G.noffset;
-      Rg.sj = G.sj;
-      Rg.sk = G.sk;
-      for (int a = 0; a < 3; a++) {
-        Rg.lo[a] = G.lo[a];
-        Rg.hi[a] = G.hi[a];
-      }
-      J.blk0[J.n++] = blk;
-      blk += ntiles<L>(G);
-    }
-    J.blk0[J.n] = blk;
-    if (blk == 0) continue;
-    J.xcd = g_xcd_map;
-    const unsigned grid = g_xcd_map ? (unsigned)(8 * ((blk + 7) / 8)) : (unsigned)blk;
-    z4c_rhs_tile<L, SH, NB, VEC, OCC><<<grid, NTHR, 0, st>>>(P, J, K, flag);
-    BH_HIP(hipGetLastError());
-  }
-  return BAMHIP_OK;
-}
+int tile_xcd_map() { return g_xcd_map; }
 
 // Split one box into its bulk region (>= 3 points from every edge) and the
 // slabs of its edge shell (fast parameters), or launch the generic per-point
@@ -1645,16 +655,6 @@ static int plan_box(const DevBox &B, const Z4cPtrs &P, const Z4cK &K, int *flag,
       add_region(T.sy, G, yl, yh);
       const int zl[3] = {ilo[0], ilo[1], lay[2][s][0]}, zh[3] = {ihi[0], ihi[1], lay[2][s][1]};
       add_region(T.sz, G, zl, zh);
-      // single layers: the distance to the edge along the slab normal is then
-      // uniform over a layer, and so are the stencil rules for most points
-      const int *lo3[3] = {xl, yl, zl}, *hi3[3] = {xh, yh, zh};
-      std::vector<Z4cGeo> *dst[3] = {&T.lx, &T.ly, &T.lz};
-      for (int a = 0; a < 3; a++)
-        for (int c = lo3[a][a]; c <= hi3[a][a]; c++) {
-          int l1[3] = {lo3[a][0], lo3[a][1], lo3[a][2]}, h1[3] = {hi3[a][0], hi3[a][1], hi3[a][2]};
-          l1[a] = h1[a] = c;
-          add_region(*dst[a], G, l1, h1);
-        }
     }
   } else if (need_edge) {
     G.edge_only = have_bulk ? 1 : 0;
@@ -1677,60 +677,20 @@ static int plan_box(const DevBox &B, const Z4cPtrs &P, const Z4cK &K, int *flag,
 // of regions (a level's boxes) is seen outside graph capture, each variant is
 // timed on it (one warm-up launch, then two timed with HIP events) and the
 // fastest is kept for that set.
-using RegionLists = std::vector<const std::vector<Z4cGeo> *>;
-using LaunchFn = int (*)(const Z4cPtrs &, const RegionLists &, const Z4cK &, int *, hipStream_t);
 struct Variant {
   const char *name;
   bool dma;    // LDS-DMA staging: byte offsets within a field must fit 32 bits
   bool pairs;  // 16-byte LDS-DMA units: needs 16-byte aligned element pairs
   LaunchFn fn;
 };
-template <class L, int NB, int VEC, int OCC>
-static int bulk_variant(const Z4cPtrs &P, const RegionLists &R, const Z4cK &K, int *flag, hipStream_t st) {
-  return launch_regions<L, false, NB, VEC, OCC>(P, *R[0], K, flag, st);
-}
-template <int NB, int VEC, int OCC>
-static int shell_variant(const Z4cPtrs &P, const RegionLists &R, const Z4cK &K, int *flag, hipStream_t st) {
-  int e;
-  if ((e = launch_regions<LSlabX, true, NB, VEC, OCC>(P, *R[0], K, flag, st))) return e;
-  if ((e = launch_regions<LSlabY, true, NB, VEC, OCC>(P, *R[1], K, flag, st))) return e;
-  return launch_regions<LSlabZ, true, NB, VEC, OCC>(P, *R[2], K, flag, st);
-}
-// the slabs with waves that keep one distance to the slab's face
-using LSlabXo = Lay<2, 16, 8, 2, 1>;
-using LSlabYo = Lay<16, 2, 8, 0, 2>;
-template <int NB, int VEC, int OCC>
-static int shell_ord_variant(const Z4cPtrs &P, const RegionLists &R, const Z4cK &K, int *flag, hipStream_t st) {
-  int e;
-  if ((e = launch_regions<LSlabXo, true, NB, VEC, OCC>(P, *R[0], K, flag, st))) return e;
-  if ((e = launch_regions<LSlabYo, true, NB, VEC, OCC>(P, *R[1], K, flag, st))) return e;
-  return launch_regions<LSlabZ, true, NB, VEC, OCC>(P, *R[2], K, flag, st);
-}
-template <int NB, int OCC>
-static int layer_variant(const Z4cPtrs &P, const RegionLists &R, const Z4cK &K, int *flag, hipStream_t st) {
-  int e;
-  if ((e = launch_regions<LLayX, true, NB, 1, OCC>(P, *R[3], K, flag, st))) return e;
-  if ((e = launch_regions<LLayY, true, NB, 1, OCC>(P, *R[4], K, flag, st))) return e;
-  return launch_regions<LLayZ, true, NB, 1, OCC>(P, *R[5], K, flag, st);
-}
-constexpr int kMaxVariants = 10;
-static const Variant kVariants[2][kMaxVariants] = {
-    {{"bulk 16x4x4 dma3", true, false, bulk_variant<LBulk, 3, 1, 1>},
-     {"bulk 16x4x4 reg", false, false, bulk_variant<LBulk, 0, 1, 1>},
-     {"bulk 16x4x4 dma4", true, false, bulk_variant<LBulk, 4, 1, 1>},
-     {"bulk 32x4x2 dma3", true, false, bulk_variant<Lay<32, 4, 2>, 3, 1, 1>},
-     {"bulk 16x8x2 dma3", true, false, bulk_variant<Lay<16, 8, 2>, 3, 1, 1>},
-     {"bulk 16x4x4 dma3 x4", true, true, bulk_variant<LBulk, 3, 4, 1>},
-     {"bulk 16x4x4 dma4 x4", true, true, bulk_variant<LBulk, 4, 4, 1>},
-     {"bulk 32x4x2 dma3 x4", true, true, bulk_variant<Lay<32, 4, 2>, 3, 4, 1>},
-     {"bulk 16x4x4 dma4 occ2", true, false, bulk_variant<LBulk, 4, 1, 2>}},
-    {{"shell layers dma3", true, false, layer_variant<3, 1>},
-     {"shell slabs reg", false, false, shell_variant<0, 1, 1>},
-     {"shell slabs dma3", true, false, shell_variant<3, 1, 1>},
-     {"shell layers dma4", true, false, layer_variant<4, 1>},
-     {"shell slabs dma3 x4", true, true, shell_variant<3, 4, 1>},
-     {"shell slabs ord dma3 x4", true, true, shell_ord_variant<3, 4, 1>}}};
-static const int kNumVariants[2] = {9, 6};
+constexpr int kMaxVariants = 3;
+static const Variant kVariants[2][kMaxVariants] = {{{"bulk 16x4x4 dma3", true, false, tile_bulk_dma},
+                                                    {"bulk 16x4x4 reg", false, false, tile_bulk_reg},
+                                                    {"bulk 16x4x4 dma3 x4", true, true, tile_bulk_dma_x4}},
+                                                   {{"shell slabs dma3", true, false, tile_shell_dma},
+                                                    {"shell slabs reg", false, false, tile_shell_reg},
+                                                    {"shell slabs dma3 x4", true, true, tile_shell_dma_x4}}};
+static const int kNumVariants[2] = {3, 3};
 // variant 0 of each kind is the default; variant 1 needs no LDS-DMA
 
 struct TuneEntry {
@@ -1830,9 +790,22 @@ static int run_rhs(bamhip_level *lev, const Z4cPtrs &P, const Z4cK &K, bool chec
   if (check_finite) set_int<<<1, 1, 0, stream()>>>(lev->d_flag, 0);
   const bool fast = (K.order_centered == 4 && K.order_advection == 4 && K.lopsided == 1 &&
                      (K.order_dissipation == 4 || K.order_dissipation == 0));
+  // The tile kernel stores a field's result while later fields' operands are
+  // still to be loaded, so an output may alias the operands of its own field
+  // only; lists crossed any other way go through the per-point kernel, which
+  // loads every operand before its first store.
+  bool crossed = false;
+  for (int v = 0; v < 25; v++)
+    for (int w = 0; w < 25; w++)
+      if (v != w)
+        for (const double *o : {(const double *)P.r[v], (const double *)P.c[v], (const double *)P.cp[v]})
+          crossed = crossed || (o && (o == P.a[w] || ((K.rk || K.addlinear) && o == P.p[w])));
   LevelTiles T;
-  for (const DevBox &B : lev->boxes)
-    if ((e = plan_box(B, P, K, lev->d_flag, fast, T))) return e;
+  for (const DevBox &B : lev->boxes) {
+    // a tile's points (at most 8 planes) within a 32-bit byte offset
+    const bool near32 = (long)B.m * B.n * 8 * 8 < 0xfffffff0L;
+    if ((e = plan_box(B, P, K, lev->d_flag, fast && !crossed && near32, T))) return e;
+  }
   // repeated launches (tuning) give the same result unless the kernels write
   // what they read
   bool repeatable = !K.rk;
@@ -1853,7 +826,7 @@ static int run_rhs(bamhip_level *lev, const Z4cPtrs &P, const Z4cK &K, bool chec
     repeatable = true;
   }
   const bool dma_ok = (long)lev->npoints * 8 < (1L << 32);
-  const RegionLists RB = {&T.bulk}, RS = {&T.sx, &T.sy, &T.sz, &T.lx, &T.ly, &T.lz};
+  const RegionLists RB = {&T.bulk}, RS = {&T.sx, &T.sy, &T.sz};
   const bool have_shell = !T.sx.empty() || !T.sy.empty() || !T.sz.empty();
   int ib = -1, is = -1;
   bool db = false, ds = false;

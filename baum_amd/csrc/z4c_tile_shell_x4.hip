@@ -1,0 +1,10 @@
+// z4c_tile_shell_x4.hip -- variants of the Z4c tile kernel (z4c_tile.h).
+#include "z4c_tile.h"
+
+namespace bamhip {
+
+int tile_shell_dma_x4(const Z4cPtrs &P, const RegionLists &R, const Z4cK &K, int *flag, hipStream_t st) {
+  return shell_variant<3, 4, 1>(P, R, K, flag, st);
+}
+
+}  // namespace bamhip

@@ -1,0 +1,151 @@
+"""The Z4c tile kernel where its tiles, its store variants and its list rules
+can go wrong.
+
+The tile kernel computes 16x4x4 tiles in the bulk and slabs two points thick
+along the box faces; a result is stored as the right-hand side, as unew =
+upre + c RHS, or as one of the RK4 stage forms.  The right-hand side is
+compared with the CPU oracle at 1e-12 of each field's largest value, as in the
+other right-hand side tests, or at the rounding floor of its second differences
+where that is larger: fields of size max|u|, each rounded by eps and weighted
+by at most 64 / 12 per h^2 (the 4th-order row -1 16 -30 16 -1 over 12), leave
+5.4 eps max|u| / h^2 a term; some of the small boxes' right-hand sides are no
+larger than 1e-3 and their terms are of order one.  The other forms with the sums formed on the host
+from the device's own right-hand side: one product and one sum, of which the
+device may fuse the product (one rounding of the product, eps |w RHS|).
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import baum_amd as B
+import oracle as O
+from spacetimes import grid, puncture_z4c
+
+pytestmark = pytest.mark.gpu
+
+EPS = np.finfo(float).eps
+U, R, A, P, ACC, V, CP = (list(range(25 * k, 25 * k + 25)) for k in range(7))
+# one tile and less, one more than a tile in each direction, only shell, slabs longer than a tile
+SIZES = [(7, 7, 7), (22, 10, 10), (23, 11, 9), (24, 14, 15), (39, 8, 21), (6, 5, 18)]
+
+
+def _level(size, seed=0):
+    h = 0.2
+    ob = O.make_box(*size, -1.9, -0.7, -0.8, h, skip=(1,) * 6)
+    X = grid(ob)
+    u = puncture_z4c(X, masses=((1.0, (0.05, -0.02, 0.03)),))
+    rng = np.random.default_rng(seed)
+    u[19:22] = 0.1 * rng.standard_normal((3,) + X.shape[1:])
+    u[13] = 0.05 * np.sin(X[0]) * np.cos(X[1])
+    u[22:25] = 0.01 * rng.standard_normal((3,) + X.shape[1:])
+    lev = B.Level([B.make_box(*size, ob.x0, ob.y0, ob.z0, h)], 175)
+    lev.enable(range(175))
+    for v in range(175):
+        lev.fill(v, 0.0)
+    lev.put_state(U, u.reshape(25, -1))
+    return lev, ob, u
+
+
+def _stage(lev, par, src, acc, accout, base, vout, copy, wc, wv):
+    L = B.lib()
+    ip = C.POINTER(C.c_int)
+    L.bamhip_z4c_rhs_rk4_stage.restype = C.c_int
+    L.bamhip_z4c_rhs_rk4_stage.argtypes = [C.c_void_p, C.POINTER(B.Z4cParams)] + [ip] * 6 + [C.c_double] * 2 + [ip]
+    arr = lambda x: None if x is None else (C.c_int * 25)(*x)  # noqa: E731
+    B.check(L.bamhip_z4c_rhs_rk4_stage(lev.h, C.byref(par), arr(src), arr(acc), arr(accout), arr(base), arr(vout),
+                                       arr(copy), wc, wv, None), "bamhip_z4c_rhs_rk4_stage")
+
+
+def _computed(size):
+    m = np.zeros(size[::-1], bool)
+    m[1:-1, 1:-1, 1:-1] = True
+    return m.reshape(-1)
+
+
+@pytest.mark.parametrize("size", SIZES)
+@pytest.mark.parametrize("params", [dict(), dict(z4_shift="withB gamma0 withGadv withBadv withShiftadv",
+                                                 z4_shiftalphapower=1.0, z4_kappa1=0.02, z4_lapse="1+log2 withshift")])
+def test_rhs_of_partial_tiles_matches_oracle(size, params):
+    lev, ob, u = _level(size)
+    cpu, _ = O.z4c_rhs(ob, O.z4c_params(**params), u)
+    lev.z4c_rhs(B.z4c_params(**params), R, U)
+    got = lev.get_state(R).reshape(u.shape)
+    floor = 64 / 12 * EPS * np.abs(u).max() / ob.dx ** 2
+    for v in range(25):
+        assert np.abs(got[v] - cpu[v]).max() <= max(1e-12 * np.abs(cpu[v]).max(), floor), B.VAR_NAMES[v]
+    lev.free()
+
+
+@pytest.mark.parametrize("size", SIZES)
+@pytest.mark.parametrize("has_v,has_cp", [(True, True), (True, False), (False, False), (False, True)])
+def test_stage_forms_match_sums_of_the_rhs(size, has_v, has_cp):
+    lev, _, u = _level(size)
+    par = B.z4c_params()
+    lev.z4c_rhs(par, R, U)
+    k = lev.get_state(R)
+    rng = np.random.default_rng(3)
+    acc, base = rng.standard_normal(k.shape), rng.standard_normal(k.shape)
+    lev.put_state(ACC, acc)
+    lev.put_state(P, base)
+    wc, wv = 0.3, 0.7
+    _stage(lev, par, U, ACC, A, P, V if has_v else None, CP if has_cp else None, wc, wv)
+    on = _computed(size)
+    for lst, want, w in ((A, acc + wc * k, wc), (V, base + wv * k, wv), (CP, base, 0.0)):
+        got = lev.get_state(lst)
+        if (lst is V and not has_v) or (lst is CP and not has_cp):
+            assert not got.any()
+            continue
+        assert not got[:, ~on].any()
+        bar = EPS * (np.abs(w * k) + np.abs(want))
+        assert (np.abs(got - want)[:, on] <= bar[:, on]).all()
+    lev.free()
+
+
+@pytest.mark.parametrize("size", SIZES)
+def test_addlinear_projects_the_sum(size):
+    """unew = upre + c RHS with the trace of At removed and det gt = 1"""
+    lev, ob, u = _level(size)
+    c = 0.05
+    par = B.z4c_params()
+    lev.put_state(P, u.reshape(25, -1))
+    lev.z4c_rhs(par, R, U, upre=P, c=c)
+    got = lev.get_state(R)
+    lev.z4c_rhs(par, A, U)
+    raw = u.reshape(25, -1) + c * lev.get_state(A)
+    on = _computed(size)
+    g, At = raw[0:6, on], raw[7:13, on]
+    det = g[0] * (g[3] * g[5] - g[4] ** 2) - g[1] * (g[1] * g[5] - g[4] * g[2]) + g[2] * (g[1] * g[4] - g[3] * g[2])
+    ig = np.array([g[3] * g[5] - g[4] ** 2, g[2] * g[4] - g[1] * g[5], g[1] * g[4] - g[2] * g[3],
+                   g[0] * g[5] - g[2] ** 2, g[1] * g[2] - g[0] * g[4], g[0] * g[3] - g[1] ** 2]) / det
+    tr = (ig * At * np.array([1, 2, 2, 1, 2, 1])[:, None]).sum(0)
+    want = raw[:, on].copy()
+    want[7:13] = At - tr / 3 * g
+    want[0:6] = g * det ** (-1 / 3)
+    for v in range(25):
+        assert np.abs(got[v][on] - want[v]).max() <= 1e-13 * max(np.abs(want[v]).max(), np.abs(raw[v]).max(), 1e-30)
+    assert not got[:, ~on].any()
+    lev.free()
+
+
+def test_lists_crossed_between_fields():
+    """an output that is another field's accumulator or start state: every
+    operand is read before any output is written"""
+    size = (24, 14, 15)
+    par = B.z4c_params()
+    rng = np.random.default_rng(5)
+    out = []
+    for crossed in (False, True):
+        lev, _, _ = _level(size)
+        acc, base = rng.standard_normal((2, 25, lev.npoints)) if not out else (out[0][2], out[0][3])
+        lev.put_state(ACC, acc)
+        lev.put_state(P, base)
+        # the next state of field v goes where the start state of field v + 1 was
+        vout = [P[(v + 1) % 25] for v in range(25)] if crossed else V
+        _stage(lev, par, U, ACC, A, P, vout, None, 0.3, 0.7)
+        out.append((lev.get_state(A), lev.get_state(vout), acc, base))
+        lev.free()
+    on = _computed(size)
+    for x, y in zip(out[0][:2], out[1][:2]):
+        scale = np.abs(x[:, on]).max(axis=1, keepdims=True)
+        assert (np.abs(x - y)[:, on] <= 1e-12 * scale).all()
