@@ -9,20 +9,12 @@
 // only two or more points away): src/main/amr/bam_amr_loops_box.h:186-215.
 //
 // Layout: SoA, one double array per grid function, ijk = i + m*j + m*n*k
-// within a box, boxes concatenated at noffset.  One thread per grid point;
-// a block is a 64 x 4 x 1 tile (one wave per x-row of 64 points, so every
-// x-neighbour load is a coalesced 512 B transaction and y/z neighbours are
-// served from L1/L2).  The algebra is ordered so that derivative groups are
-// consumed as soon as they are formed (second derivatives of gt go straight
-// into the Ricci accumulators, those of beta into the Gamma-driver terms),
-// keeping the live FP64 state within the VGPR budget of one wave per SIMD.
+// within a box, boxes concatenated at noffset.
 //
-// Two derivative providers share the algebra:
-//   Bulk4 : points >= 3 away from every box edge, 4th-order centred
-//           stencils, lop-sided (offset 1) 4th-order advection;
-//   Edge  : any point, with the reference's per-point order selection,
-//           used for the shell of points 1 and 2 away from the box edge and
-//           for parameter choices other than (4, 4, lop-sided 1).
+// The usual parameters (order 4, lop-sided 1) run in the tile kernel of
+// z4c_tile.h, planned and launched here.  Any other choice runs in the per-point
+// kernel below, whose derivative provider follows the reference's order
+// selection point by point.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -670,9 +662,8 @@ static int plan_box(const DevBox &B, const Z4cPtrs &P, const Z4cK &K, int *flag,
 }
 
 // ---- autotuner of the tile kernels
-// A variant is one instantiation of the tile kernel: tile shape (TX x TY x
-// TZ, so the z depth of a block) and staging (registers, or LDS-DMA with NB
-// buffers).  Every variant evaluates the same per-point arithmetic in the same
+// A variant is one staging of the tile kernel: through registers, or by
+// LDS-DMA in dwords or in 16-byte units.  Every variant evaluates the same per-point arithmetic in the same
 // order, so all give bitwise the same right-hand side.  The first time a set
 // of regions (a level's boxes) is seen outside graph capture, each variant is
 // timed on it (one warm-up launch, then two timed with HIP events) and the
@@ -684,12 +675,12 @@ struct Variant {
   LaunchFn fn;
 };
 constexpr int kMaxVariants = 3;
-static const Variant kVariants[2][kMaxVariants] = {{{"bulk 16x4x4 dma3", true, false, tile_bulk_dma},
-                                                    {"bulk 16x4x4 reg", false, false, tile_bulk_reg},
-                                                    {"bulk 16x4x4 dma3 x4", true, true, tile_bulk_dma_x4}},
-                                                   {{"shell slabs dma3", true, false, tile_shell_dma},
-                                                    {"shell slabs reg", false, false, tile_shell_reg},
-                                                    {"shell slabs dma3 x4", true, true, tile_shell_dma_x4}}};
+static const Variant kVariants[2][kMaxVariants] = {{{"bulk 16x4x4 dma3", true, false, tile_dma},
+                                                    {"bulk 16x4x4 reg", false, false, tile_reg},
+                                                    {"bulk 16x4x4 dma3 x4", true, true, tile_dma_x4}},
+                                                   {{"shell slabs dma3", true, false, tile_dma},
+                                                    {"shell slabs reg", false, false, tile_reg},
+                                                    {"shell slabs dma3 x4", true, true, tile_dma_x4}}};
 static const int kNumVariants[2] = {3, 3};
 // variant 0 of each kind is the default; variant 1 needs no LDS-DMA
 
@@ -698,7 +689,7 @@ struct TuneEntry {
   double ms[kMaxVariants];
 };
 struct TuneState {
-  int overlap = 1;  // shell on the side stream, concurrent with the bulk
+  int overlap = 1;  // shell and bulk tiles in one launch
   int mode = 1;  // 0: defaults only; 1: tune each new region set
   int forced[2] = {-1, -1};
   std::map<std::string, TuneEntry> chosen[2];
@@ -708,8 +699,9 @@ static TuneState g_tune;
 static std::string region_signature(const RegionLists &R) {
   std::string s;
   char buf[96];
-  for (const auto *v : R) {
+  for (const auto *v : R.kind) {
     s += '|';
+    if (!v) continue;
     for (const Z4cGeo &G : *v) {
       snprintf(buf, sizeof buf, "%d,%d,%d:%d-%d,%d-%d,%d-%d;", G.m, G.n, G.o, G.lo[0], G.hi[0], G.lo[1], G.hi[1],
                G.lo[2], G.hi[2]);
@@ -826,7 +818,8 @@ static int run_rhs(bamhip_level *lev, const Z4cPtrs &P, const Z4cK &K, bool chec
     repeatable = true;
   }
   const bool dma_ok = (long)lev->npoints * 8 < (1L << 32);
-  const RegionLists RB = {&T.bulk}, RS = {&T.sx, &T.sy, &T.sz};
+  const RegionLists RB = {{&T.bulk, nullptr, nullptr, nullptr}}, RS = {{nullptr, &T.sx, &T.sy, &T.sz}},
+                    RA = {{&T.bulk, &T.sx, &T.sy, &T.sz}};
   const bool have_shell = !T.sx.empty() || !T.sy.empty() || !T.sz.empty();
   int ib = -1, is = -1;
   bool db = false, ds = false;
@@ -841,16 +834,10 @@ static int run_rhs(bamhip_level *lev, const Z4cPtrs &P, const Z4cK &K, bool chec
   if (have_shell && (e = choose_variant(1, PT, RS, KT, lev->d_flag, repeatable, dma_ok, pairs_ok, &is, &ds)))
     return e;
   if (K.rk) db = ds = false;  // the tuner ran the plain RHS; the stage itself is still to run
-  if (ib >= 0 && is >= 0 && !db && !ds && g_tune.overlap) {
-    // the shell on the side stream beside the bulk: the two write disjoint
-    // points, and the shell's few blocks fill the CUs the bulk's last wave of
-    // blocks leaves idle.  The bulk is enqueued first (1% faster on the FMR
-    // hierarchy than the shell first).
+  if (ib >= 0 && is >= 0 && !db && !ds && g_tune.overlap && kVariants[0][ib].fn == kVariants[1][is].fn) {
+    // bulk and slabs staged the same way: one launch
     TimerScope t("z4_rhs");
-    if ((e = fork_side())) return e;
-    if ((e = kVariants[0][ib].fn(P, RB, K, lev->d_flag, stream()))) return e;
-    if ((e = kVariants[1][is].fn(P, RS, K, lev->d_flag, side_stream()))) return e;
-    if ((e = join_side())) return e;
+    if ((e = kVariants[0][ib].fn(P, RA, K, lev->d_flag, stream()))) return e;
   } else {
     if (ib >= 0 && !db) {
       TimerScope t("z4_rhs");

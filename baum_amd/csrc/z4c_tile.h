@@ -86,7 +86,7 @@ __device__ __forceinline__ constexpr int mixid(int a, int b) {  // xy=0 xz=1 yz=
   return (a + b) - 1;
 }
 
-// ------------------------------------------------------- bulk kernel (LDS)
+// ------------------------------------------------------- tile kernel (LDS)
 // Output tile of TX x TY x TZ points per block (256 threads, one point per
 // thread).  Each of the 25 grid functions is staged in turn into an LDS tile
 // with a halo of 3 points (the reach of the lop-sided advection stencil), so
@@ -98,43 +98,23 @@ __device__ __forceinline__ constexpr int mixid(int a, int b) {  // xy=0 xz=1 yz=
 // 2 x 16 x 8, 16 x 2 x 8 and 16 x 8 x 2 on the x, y and z faces.
 constexpr int HALO = 3;
 constexpr int NTHR = 256;
-// PX: unused LDS columns at the end of each tile row (the row stride SX is
-// the staged width WX plus PX), chosen so that the 16 lanes of a read phase
-// fall on distinct banks
-// ORD: which point of the tile thread t of the block computes (64 threads
-// form a wave): 0, x fastest, then y, then z; 1, y fastest, then z, then x
-// (a wave keeps one x, as the layers of an x-face slab do); 2, x fastest,
-// then z, then y (a wave keeps one y).
-template <int TX_, int TY_, int TZ_, int PX = 0, int ORD = 0>
+template <int TX_, int TY_, int TZ_>
 struct Lay {
   static constexpr int TX = TX_, TY = TY_, TZ = TZ_;
-  static constexpr int WX = TX + 2 * HALO;
-  static constexpr int SX = WX + PX, SY = TY + 2 * HALO, SZ = TZ + 2 * HALO;
+  static constexpr int SX = TX + 2 * HALO, SY = TY + 2 * HALO, SZ = TZ + 2 * HALO;
   static constexpr int TILE = SX * SY * SZ;
   static constexpr int NLOAD = (TILE + NTHR - 1) / NTHR;
   static_assert(TX * TY * TZ == NTHR, "one point per thread");
-  static_assert(ORD >= 0 && ORD <= 2, "thread order");
   __device__ static void coords(int t, int &x, int &y, int &z) {
-    if constexpr (ORD == 1) {
-      y = t % TY;
-      z = (t / TY) % TZ;
-      x = t / (TY * TZ);
-    } else if constexpr (ORD == 2) {
-      x = t % TX;
-      z = (t / TX) % TZ;
-      y = t / (TX * TZ);
-    } else {
-      x = t % TX;
-      y = (t / TX) % TY;
-      z = t / (TX * TY);
-    }
+    x = t % TX;
+    y = (t / TX) % TY;
+    z = t / (TX * TY);
   }
 };
 using LBulk = Lay<16, 4, 4>;
-// x faces: rows of 2 points, so without padding (stride 8 doubles) the
-// lanes (x, y) = (0..1, 0..7) of a read phase meet on 4 banks; a stride of 10
-// spreads them over all 32
-using LSlabX = Lay<2, 16, 8, 2>;
+// x faces: rows of 2 points.  (Rows padded from 8 to 10 doubles spread the lanes
+// of a read phase over all banks, but take 98 KB of LDS, so one block per CU.)
+using LSlabX = Lay<2, 16, 8>;
 using LSlabY = Lay<16, 2, 8>;
 using LSlabZ = Lay<16, 8, 2>;
 
@@ -374,7 +354,7 @@ struct Stager {
       const int idx = tid + k * NTHR;
       const int x = idx % L::SX, y = (idx / L::SX) % L::SY, z = idx / (L::SX * L::SY);
       const int gi = i0 - HALO + x, gj = j0 - HALO + y, gk = k0 - HALO + z;
-      const bool in = idx < L::TILE && x < L::WX && gi >= 0 && gj >= 0 && gk >= 0 && gi < G.m && gj < G.n && gk < G.o;
+      const bool in = idx < L::TILE && gi >= 0 && gj >= 0 && gk >= 0 && gi < G.m && gj < G.n && gk < G.o;
       goff[k] = in ? (int)(x + G.sj * y + G.sk * z) : 0;
       ok |= in ? (1u << k) : 0u;
     }
@@ -427,7 +407,7 @@ struct DmaStager {
       const int e = VEC == 1 ? d >> 1 : 2 * d;
       const int x = e % L::SX, y = (e / L::SX) % L::SY, z = e / (L::SX * L::SY);
       const int gi = i0 - HALO + x, gj = j0 - HALO + y, gk = k0 - HALO + z;
-      const bool in = e < L::TILE && x < L::WX;
+      const bool in = e < L::TILE;
       // clamped into the box; for 16-byte units gi is even and so is the
       // box's row length, so the clamped pair is (0, 1) or (m - 2, m - 1)
       const int ci = min(max(gi, 0), G.m - (VEC == 1 ? 1 : 2)), cj = min(max(gj, 0), G.n - 1),
@@ -481,18 +461,21 @@ __device__ __forceinline__ void pin(double (&a)[N]) {
 // The grid spacing constants are common to the regions of one launch (one
 // level), so a region carries only integer geometry.
 constexpr int kMaxRegions = 32;
+// kind: the tile layout, 0 bulk, 1 to 3 slabs normal to x, y and z
 struct RegionGeo {
   long noffset;
   int m, n, o;
   int lo[3], hi[3];
+  int kind;
 };
 struct Spacing {
-  double h[3], ih[3], i12h[3], i12hh[3], i144hh[3], i2h[3], ihh[3], i4hh[3];
+  double h[3], ih[3], i12h[3], i12hh[3], i144hh[3];
 };
 struct TileJobs {
   int n;
   int blk0[kMaxRegions + 1];  // first tile of each region; blk0[n] = number of tiles
-  int xcd;                    // 1: XCD-aware numbering of the tiles (grid padded to a multiple of 8)
+  int nshell;                 // tiles of the slabs, which come before the bulk's
+  int xcd;                    // 1: XCD-aware numbering of the tiles (grid padded)
   RegionGeo reg[kMaxRegions];
   Spacing sp;
 };
@@ -508,8 +491,13 @@ struct TilePtrs {
   StagePtrs gam[3];       // Gamma^i: operands and outputs
   const double *u[BAMHIP_Z4C_NVARS];  // by field, for the point values
 };
-static_assert(sizeof(TilePtrs) + sizeof(TileJobs) + sizeof(Z4cK) + sizeof(int *) <= 4096,
-              "arguments of the tile kernel within 4 KiB");
+struct TileArgs {
+  TilePtrs P;
+  TileJobs J;
+  Z4cK K;
+  int *flag;
+};
+static_assert(sizeof(TileArgs) <= 4096, "arguments of the tile kernel within 4 KiB");
 
 // What a result is stored as: the right-hand side; upre + c RHS with the
 // projection; or an RK4 stage's accumulator with (V) the next state and (C)
@@ -573,31 +561,30 @@ struct StageBuf<L, 0, VEC> {
   static constexpr int n = L::TILE;
 };
 
-// NB = 0: one LDS tile, staged through registers (Stager); NB >= 2: NB LDS
-// buffers filled by the LDS-DMA path (DmaStager).  OCC: blocks per CU the
-// register allocation must allow (2 caps a thread at 256 registers, with
-// spills, for two waves per SIMD).
-template <class L, bool SH, class ST, int NB, int VEC, int OCC>
-__global__ void __launch_bounds__(NTHR, OCC) z4c_rhs_tile(TilePtrs P, TileJobs J, Z4cK K, int *flag) {
-  // the staging buffers, then per thread six values of the Gamma^i stages
-  // that are needed again at the end.  One array: with two, the compiler tells
-  // LDS objects apart and waits for every transfer before each stage's reads
-  __shared__ double tile[StageBuf<L, NB, VEC>::n + 6 * NTHR];
+// LDS of a block: the staging buffers, then per thread six values of the
+// Gamma^i stages that are needed again at the end.  One array: with two, the
+// compiler tells LDS objects apart and waits for every transfer before each
+// stage's reads.
+template <class L, int NB, int VEC>
+constexpr int tile_lds() {
+  return StageBuf<L, NB, VEC>::n + 6 * NTHR;
+}
+
+// One tile, number b of region r.  NB = 0: one LDS tile, staged through
+// registers (Stager); NB >= 2: NB LDS buffers filled by the LDS-DMA path
+// (DmaStager).
+template <class L, bool SH, class ST, int NB, int VEC>
+__device__ __forceinline__ void tile_body(double *tile, int r, int b) {
+  // the kernel's arguments, read anew by each layout's body: shared, the
+  // compiler loads them all ahead of the branch on the layout and spills
+  // hundreds of scalar registers
+  auto *ka = (const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(ka));
+  const TileArgs &args = *(const TileArgs *)ka;
+  const TilePtrs &P = args.P;
+  const TileJobs &J = args.J;
+  const Z4cK &K = args.K;
   double *const park = tile + StageBuf<L, NB, VEC>::n;
-  // Tile of this block.  Workgroups are dispatched to the 8 XCDs round-robin
-  // (workgroup w to XCD w mod 8), each XCD with its own L2.  With xcd set,
-  // workgroup w takes tile (w mod 8) * per + w / 8, so every XCD works through
-  // one contiguous range of tiles and neighbouring tiles, which stage the same
-  // halo points, meet in the same L2.
-  int t = (int)blockIdx.x;
-  if (J.xcd) {
-    const int per = (int)gridDim.x / 8;
-    t = (t % 8) * per + t / 8;
-    if (t >= J.blk0[J.n]) return;  // padding workgroup (whole block, before any barrier)
-  }
-  // region of this block (uniform): the regions' tiles are numbered in order
-  int r = 0;
-  while (r + 1 < J.n && t >= J.blk0[r + 1]) r++;
   // copies: indexing the argument array by r through a reference would stage it in scratch
   const RegionGeo Rg = J.reg[r];
   Z4cGeo G;
@@ -616,12 +603,8 @@ __global__ void __launch_bounds__(NTHR, OCC) z4c_rhs_tile(TilePtrs P, TileJobs J
     G.i12h[a] = J.sp.i12h[a];
     G.i12hh[a] = J.sp.i12hh[a];
     G.i144hh[a] = J.sp.i144hh[a];
-    G.i2h[a] = J.sp.i2h[a];
-    G.ihh[a] = J.sp.ihh[a];
-    G.i4hh[a] = J.sp.i4hh[a];
   }
   G.edge_only = 0;
-  const int b = t - J.blk0[r];
   const int ntx = (G.hi[0] - G.lo[0] + L::TX) / L::TX, nty = (G.hi[1] - G.lo[1] + L::TY) / L::TY;
   const int tid = (int)threadIdx.x;
   int tx, ty, tz;
@@ -1087,8 +1070,47 @@ __global__ void __launch_bounds__(NTHR, OCC) z4c_rhs_tile(TilePtrs P, TileJobs J
   });
   flush(E[24 % 2], P.st[25]);
   if (!active) return;
-  if (bad) *flag = 1;
+  if (bad) *args.flag = 1;
   if constexpr (ST::ADD) project_point(P, K, qb + loc / 8);
+}
+
+// The right-hand side of a level: slab and bulk tiles of all its boxes in one
+// launch.  (As one launch for the bulk and one per slab orientation on a second
+// stream, the slabs' few blocks, each as long as any other, ran one orientation
+// after another and ended the evaluation: 24^3 box 0.11 ms, 64^3 0.16 ms.)
+// The slab tiles come first, so that none is left to the end.  Two blocks per
+// CU: 80 KB of LDS and 256 registers each.  SLABS = false: bulk regions only, as
+// of a periodic box (the kernel of all four bodies spills 20 more registers:
+// 2.42 instead of 2.24 ms on 192^3).
+//
+// Workgroups are dispatched to the 8 XCDs round-robin (workgroup w to XCD w mod
+// 8), each XCD with its own L2.  With xcd set, each XCD takes one contiguous
+// range of the slab tiles and one of the bulk tiles, so that neighbouring tiles,
+// which stage the same halo points, meet in the same L2.
+template <class ST, int NB, int VEC, bool SLABS>
+__global__ void __launch_bounds__(NTHR, 2) z4c_rhs_tile(TileArgs args) {
+  constexpr int n0 = tile_lds<LBulk, NB, VEC>(), n1 = tile_lds<LSlabX, NB, VEC>(), n2 = tile_lds<LSlabY, NB, VEC>(),
+                n3 = tile_lds<LSlabZ, NB, VEC>();
+  constexpr int nl = (n0 > n1 ? n0 : n1) > (n2 > n3 ? n2 : n3) ? (n0 > n1 ? n0 : n1) : (n2 > n3 ? n2 : n3);
+  static_assert(nl * sizeof(double) <= 80 * 1024, "two blocks per CU");
+  __shared__ double tile[nl];
+  const TileJobs &J = args.J;
+  int t = (int)blockIdx.x;
+  if (J.xcd) {
+    const int per = (J.nshell + 7) / 8, perb = (J.blk0[J.n] - J.nshell + 7) / 8, x = t % 8, i = t / 8;
+    const bool shell = i < per;
+    t = shell ? x * per + i : J.nshell + x * perb + (i - per);
+    // padding workgroup (whole block, before any barrier)
+    if (t >= (shell ? J.nshell : J.blk0[J.n])) return;
+  }
+  // region of this block (uniform): the regions' tiles are numbered in order
+  int r = 0;
+  while (r + 1 < J.n && t >= J.blk0[r + 1]) r++;
+  const int b = t - J.blk0[r], kind = SLABS ? J.reg[r].kind : 0;
+  if (kind == 0) tile_body<LBulk, false, ST, NB, VEC>(tile, r, b);
+  else if (kind == 1) tile_body<LSlabX, true, ST, NB, VEC>(tile, r, b);
+  else if (kind == 2) tile_body<LSlabY, true, ST, NB, VEC>(tile, r, b);
+  else tile_body<LSlabZ, true, ST, NB, VEC>(tile, r, b);
 }
 
 // XCD-aware tile numbering on (bamhip_z4c_set_xcd_map)
@@ -1105,9 +1127,22 @@ inline bool same_spacing(const Z4cGeo &a, const Z4cGeo &b) {
 }
 
 // one launch per kMaxRegions regions of a layout (and per grid spacing)
-template <class L, bool SH, int NB, int VEC, int OCC>
-int launch_regions(const Z4cPtrs &F, const std::vector<Z4cGeo> &regs, const Z4cK &K, int *flag,
-                          hipStream_t st) {
+// regions of one level by layout: the bulk, and slabs normal to x, y and z
+struct RegionLists {
+  const std::vector<Z4cGeo> *kind[4];  // null: none of that kind
+};
+template <int NB, int VEC>
+int launch_tiles(const Z4cPtrs &F, const RegionLists &R, const Z4cK &K, int *flag, hipStream_t st) {
+  struct Reg {
+    const Z4cGeo *g;
+    int kind;
+  };
+  std::vector<Reg> regs;
+  // grouped so that a launch's slabs come before its bulk regions and a level
+  // of few boxes is one launch
+  for (int kind : {1, 2, 3, 0})
+    if (R.kind[kind])
+      for (const Z4cGeo &G : *R.kind[kind]) regs.push_back({&G, kind});
   constexpr int LEAD = NB == 0 ? 1 : NB - 1;
   TilePtrs P{};
   for (int v = 0; v < 25; v++) P.u[v] = F.u[v];
@@ -1133,22 +1168,21 @@ int launch_regions(const Z4cPtrs &F, const std::vector<Z4cGeo> &regs, const Z4cK
   size_t r0 = 0;
   while (r0 < regs.size()) {
     TileJobs J{};
-    const Z4cGeo &G0 = regs[r0];
+    const Z4cGeo &G0 = *regs[r0].g;
     for (int a = 0; a < 3; a++) {
       J.sp.h[a] = G0.h[a];
       J.sp.ih[a] = G0.ih[a];
       J.sp.i12h[a] = G0.i12h[a];
       J.sp.i12hh[a] = G0.i12hh[a];
       J.sp.i144hh[a] = G0.i144hh[a];
-      J.sp.i2h[a] = G0.i2h[a];
-      J.sp.ihh[a] = G0.ihh[a];
-      J.sp.i4hh[a] = G0.i4hh[a];
     }
     int blk = 0;
     J.n = 0;
-    while (r0 < regs.size() && J.n < kMaxRegions && same_spacing(regs[r0], G0)) {
-      const Z4cGeo &G = regs[r0++];
+    while (r0 < regs.size() && J.n < kMaxRegions && same_spacing(*regs[r0].g, G0)) {
+      const Z4cGeo &G = *regs[r0].g;
+      const int kind = regs[r0++].kind;
       RegionGeo &Rg = J.reg[J.n];
+      Rg.kind = kind;
       Rg.m = G.m;
       Rg.n = G.n;
       Rg.o = G.o;
@@ -1158,14 +1192,19 @@ int launch_regions(const Z4cPtrs &F, const std::vector<Z4cGeo> &regs, const Z4cK
         Rg.hi[a] = G.hi[a];
       }
       J.blk0[J.n++] = blk;
-      blk += ntiles<L>(G);
+      blk += kind == 0 ? ntiles<LBulk>(G) : kind == 1 ? ntiles<LSlabX>(G) : kind == 2 ? ntiles<LSlabY>(G)
+                                                                                        : ntiles<LSlabZ>(G);
+      if (kind) J.nshell = blk;
     }
     J.blk0[J.n] = blk;
     if (blk == 0) continue;
     J.xcd = tile_xcd_map();
-    const unsigned grid = tile_xcd_map() ? (unsigned)(8 * ((blk + 7) / 8)) : (unsigned)blk;
+    const unsigned grid = J.xcd ? (unsigned)(8 * ((J.nshell + 7) / 8 + (blk - J.nshell + 7) / 8)) : (unsigned)blk;
     auto go = [&](auto st_) {
-      z4c_rhs_tile<L, SH, decltype(st_), NB, VEC, OCC><<<grid, NTHR, 0, st>>>(P, J, K, flag);
+      if (J.nshell)
+        z4c_rhs_tile<decltype(st_), NB, VEC, true><<<grid, NTHR, 0, st>>>(TileArgs{P, J, K, flag});
+      else
+        z4c_rhs_tile<decltype(st_), NB, VEC, false><<<grid, NTHR, 0, st>>>(TileArgs{P, J, K, flag});
     };
     if (!K.rk) {
       if (K.addlinear) go(StoreAs<false, true, false, false>{});
@@ -1182,26 +1221,10 @@ int launch_regions(const Z4cPtrs &F, const std::vector<Z4cGeo> &regs, const Z4cK
   return BAMHIP_OK;
 }
 
-// regions of one level by layout, and the launchers of the tile kernel's
-// variants over them (z4c_tile_*.hip): R holds the bulk, or the x, y and z slabs
-using RegionLists = std::vector<const std::vector<Z4cGeo> *>;
+// launchers of the staging variants, one per file (z4c_tile_*.hip)
 using LaunchFn = int (*)(const Z4cPtrs &, const RegionLists &, const Z4cK &, int *, hipStream_t);
-template <class L, int NB, int VEC, int OCC>
-int bulk_variant(const Z4cPtrs &P, const RegionLists &R, const Z4cK &K, int *flag, hipStream_t st) {
-  return launch_regions<L, false, NB, VEC, OCC>(P, *R[0], K, flag, st);
-}
-template <int NB, int VEC, int OCC>
-int shell_variant(const Z4cPtrs &P, const RegionLists &R, const Z4cK &K, int *flag, hipStream_t st) {
-  int e;
-  if ((e = launch_regions<LSlabX, true, NB, VEC, OCC>(P, *R[0], K, flag, st))) return e;
-  if ((e = launch_regions<LSlabY, true, NB, VEC, OCC>(P, *R[1], K, flag, st))) return e;
-  return launch_regions<LSlabZ, true, NB, VEC, OCC>(P, *R[2], K, flag, st);
-}
-int tile_bulk_dma(const Z4cPtrs &, const RegionLists &, const Z4cK &, int *, hipStream_t);
-int tile_bulk_reg(const Z4cPtrs &, const RegionLists &, const Z4cK &, int *, hipStream_t);
-int tile_bulk_dma_x4(const Z4cPtrs &, const RegionLists &, const Z4cK &, int *, hipStream_t);
-int tile_shell_dma(const Z4cPtrs &, const RegionLists &, const Z4cK &, int *, hipStream_t);
-int tile_shell_reg(const Z4cPtrs &, const RegionLists &, const Z4cK &, int *, hipStream_t);
-int tile_shell_dma_x4(const Z4cPtrs &, const RegionLists &, const Z4cK &, int *, hipStream_t);
+int tile_dma(const Z4cPtrs &, const RegionLists &, const Z4cK &, int *, hipStream_t);
+int tile_reg(const Z4cPtrs &, const RegionLists &, const Z4cK &, int *, hipStream_t);
+int tile_dma_x4(const Z4cPtrs &, const RegionLists &, const Z4cK &, int *, hipStream_t);
 
 }  // namespace bamhip

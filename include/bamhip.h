@@ -168,8 +168,9 @@ int bamhip_z4c_rhs(bamhip_level *lev, const bamhip_z4c_params *par,
  * i (-1: back to the tuner).  tune_report writes one line per tuned set with
  * the time of each variant and returns the length needed (with the NUL). */
 int bamhip_z4c_tune_mode(int mode);
-/* on != 0 (default): the shell kernels run on a second stream concurrently
- * with the bulk kernel (both in a captured graph too); returns the old value */
+/* on != 0 (default): the bulk and box-edge shell tiles of a level run in one
+ * launch where both are staged the same way, else one after the other; returns
+ * the old value */
 int bamhip_z4c_set_overlap(int on);
 /* on != 0 (default): the tile kernels number their tiles so that each of the
  * 8 XCDs (workgroup w runs on XCD w mod 8) takes one contiguous range of
