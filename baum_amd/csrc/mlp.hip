@@ -2,12 +2,12 @@
 // (3 -> 64 -> 64 -> 1, ReLU, bf16 weights with FP32 masters and FP32
 // accumulation, Adam) on gfx950.  No reference counterpart.
 //
-// Training step: one wavefront per 64 samples (mlp_train_kernel) runs the
-// forward pass of mlp_device.h, the MSE loss and the backward pass:
-//   dW3, db2, db3: per-feature sums over the wave's points (LDS);
+// Training step: one block per 64 samples (mlp_train_kernel) runs the forward
+// pass, the MSE loss and the backward pass:
+//   dW3, db2, db3: per-feature sums over the block's points (LDS);
 //   dW2 = dZ2 . H1 and dH1^T = W2^T . dZ2 on the matrix cores (bf16 operands,
 //   FP32 accumulate), the same 32x32x16 layout as the forward pass;
-//   dW1, db1: per-unit sums over the wave's points (LDS);
+//   dW1, db1: per-unit sums over the block's points (LDS);
 // and writes its partial gradient.  mlp_update_kernel sums the partials in a
 // fixed order (deterministic), applies Adam to the FP32 masters and refreshes
 // the bf16 working copies.
@@ -55,16 +55,27 @@ namespace {
 
 constexpr int kWave = 64;
 
-__global__ void mlp_train_kernel(MlpView M, const float *__restrict__ feat, const float *__restrict__ target, long n,
-                                 long q0, long batch, unsigned long long pa, unsigned long long pb,
-                                 float *__restrict__ part, float *__restrict__ lossp, float inv_batch) {
+// Four wavefronts per 64 samples: the batch is small (4096 samples are 64
+// blocks), so the kernel is one block's chain of latencies.  Each wavefront takes
+// 16 units of layer 1, one 32x32 tile of every contraction and 16 samples of
+// every per-feature sum; with one wavefront a block took all of them in turn
+// (16.6 us for 4096 samples, now 8.0).
+constexpr int kTrainWaves = 4;
+
+__global__ void __launch_bounds__(kWave *kTrainWaves)
+    mlp_train_kernel(MlpView M, const float *__restrict__ feat, const float *__restrict__ target, long n, long q0,
+                     long batch, unsigned long long pa, unsigned long long pb, float *__restrict__ part,
+                     float *__restrict__ lossp, float inv_batch) {
   __shared__ __attribute__((aligned(16))) __bf16 h1[kWave * kHStr];    // [pt][k]
   __shared__ __attribute__((aligned(16))) __bf16 h1t[kMlpH * kHStr];   // [k][pt]
   __shared__ __attribute__((aligned(16))) __bf16 dz2[kMlpH * kHStr];   // [f][pt]
   __shared__ __attribute__((aligned(16))) __bf16 dz2t[kWave * kHStr];  // [pt][f]
-  __shared__ float hs[kMlpH * (kWave + 1)];                            // h2 [f][pt], then dz1 [k][pt]
-  __shared__ float xsh[kWave * 3], dys[kWave];
-  const int l = threadIdx.x, lr = l % 32, lh = l / 32;
+  __shared__ float h2[kMlpH * (kWave + 1)];                            // [f][pt]
+  __shared__ float dz1[kMlpH * (kWave + 1)];                           // [k][pt]
+  __shared__ float xsh[kWave * 3], ts[kWave], dys[kWave], ysum[2][kWave];
+  __shared__ float red[kTrainWaves][7][kMlpH];  // per wave: dW3, db2, db3, dW1 (3), db1
+  const int l = threadIdx.x % kWave, w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int lr = l % 32, lh = l / 32, m = w / 2, n2 = w % 2;  // the wave's tile: rows 32m.., columns 32 n2..
   const long slot = (long)blockIdx.x * kWave + l;
   // ---- sample: a fixed affine permutation of [0, n) per epoch
   bool valid = slot < batch && q0 + slot < n;
@@ -76,146 +87,157 @@ __global__ void mlp_train_kernel(MlpView M, const float *__restrict__ feat, cons
     valid = isfinite(x[0]) && isfinite(x[1]) && isfinite(x[2]) && isfinite(t);
     if (!valid) x[0] = x[1] = x[2] = t = 0.f;
   }
-  for (int j = 0; j < 3; j++) xsh[3 * l + j] = x[j];
-  // ---- forward
-  mlp_layer1(M, x, h1 + l * kHStr);
-  for (int k = 0; k < kMlpH; k++) h1t[k * kHStr + l] = h1[l * kHStr + k];
+  if (w == 0) {
+    for (int j = 0; j < 3; j++) xsh[3 * l + j] = x[j];
+    ts[l] = valid ? t : __builtin_nanf("");
+  }
+  // ---- forward: layer 1, units 16 w .. 16 w + 15 of every point
+#pragma unroll
+  for (int k0 = 0; k0 < 16; k0 += 8) {
+    bf16x8 h;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const int k = 16 * w + k0 + e;
+      h[e] = (__bf16)fmaxf(mlp_z1(M, k, x), 0.f);
+      h1t[k * kHStr + l] = h[e];
+    }
+    *(bf16x8 *)(h1 + l * kHStr + 16 * w + k0) = h;
+  }
   __syncthreads();
-  f32x16 c[2][2];
-  const float y = mlp_layer23(M, h1, c, M.p + kOffB2, M.wq + 192);
-  const float r = valid ? y - t : 0.f;
+  // ---- layer 2: features 32m.., points 32 n2..; layer 3 summed over the features
+  f32x16 c;
+#pragma unroll
+  for (int v = 0; v < 16; v++) c[v] = 0.f;
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    const bf16x8 b = *(const bf16x8 *)(h1 + (32 * n2 + lr) * kHStr + 16 * s + 8 * lh);
+    const bf16x8 a = *(const bf16x8 *)(M.w2 + (32 * m + lr) * kMlpH + 16 * s + 8 * lh);
+    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+  }
+  float w3[16], yp = 0.f;
+#pragma unroll
+  for (int v = 0; v < 16; v++) {
+    const int f = 32 * m + mfma_row(v, l);
+    w3[v] = M.wq[192 + f];
+    c[v] = fmaxf(c[v] + M.p[kOffB2 + f], 0.f);
+    yp = fmaf(c[v], w3[v], yp);
+  }
+  yp += __shfl_xor(yp, 32);
+  if (lh == 0) ysum[m][32 * n2 + lr] = yp;
+  __syncthreads();
+  const float y = ysum[0][l] + ysum[1][l] + M.p[kOffB3], tl = ts[l];
+  const float r = isfinite(tl) ? y - tl : 0.f;
   const float dy = 2.f * r * inv_batch;
-  float lsum = r * r;
-  for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
-  if (l == 0) lossp[blockIdx.x] = lsum;
-  dys[l] = dy;
+  if (w == 0) {
+    float lsum = r * r;
+    for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
+    if (l == 0) lossp[blockIdx.x] = lsum;
+    dys[l] = dy;
+  }
   // ---- dZ2 = relu'(z2) * W3 * dy, kept as bf16 in both layouts; h2 kept in FP32
-#pragma unroll
-  for (int n2 = 0; n2 < 2; n2++) {
-    const float dyp = __shfl(dy, 32 * n2 + lr);
+  {
     const int pt = 32 * n2 + lr;
+    const float dyp = __shfl(dy, pt);
 #pragma unroll
-    for (int m = 0; m < 2; m++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) {
-        const int f = 32 * m + mfma_row(v, l);
-        const float h = c[m][n2][v];
-        const float dz = h > 0.f ? M.wq[192 + f] * dyp : 0.f;
-        hs[f * (kWave + 1) + pt] = h;
-        dz2[f * kHStr + pt] = (__bf16)dz;
-        dz2t[pt * kHStr + f] = (__bf16)dz;
-      }
+    for (int v = 0; v < 16; v++) {
+      const int f = 32 * m + mfma_row(v, l);
+      const float dz = c[v] > 0.f ? w3[v] * dyp : 0.f;
+      h2[f * (kWave + 1) + pt] = c[v];
+      dz2[f * kHStr + pt] = (__bf16)dz;
+      dz2t[pt * kHStr + f] = (__bf16)dz;
+    }
   }
   __syncthreads();
   float *g = part + (long)blockIdx.x * kMlpNParam;
   {
-    // lane f: dW3[f], db2[f]; lane 0 also db3
-    const int f = l;
-    const float w3 = M.wq[192 + f];
-    float gw3 = 0.f, gb2 = 0.f;
-    for (int pt = 0; pt < kWave; pt++) {
-      const float h = hs[f * (kWave + 1) + pt];
-      gw3 = fmaf(h, dys[pt], gw3);
-      gb2 += h > 0.f ? w3 * dys[pt] : 0.f;
+    // lane f, points 16 w ..: dW3[f], db2[f], db3
+    const float w3f = M.wq[192 + l];
+    float gw3 = 0.f, gb2 = 0.f, gb3 = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      const int pt = 16 * w + e;
+      const float h = h2[l * (kWave + 1) + pt], d = dys[pt];
+      gw3 = fmaf(h, d, gw3);
+      gb2 += h > 0.f ? w3f * d : 0.f;
+      gb3 += d;
     }
-    g[kOffW3 + f] = gw3;
-    g[kOffB2 + f] = gb2;
-    if (l == 0) {
-      float gb3 = 0.f;
-      for (int pt = 0; pt < kWave; pt++) gb3 += dys[pt];
-      g[kOffB3] = gb3;
-    }
+    red[w][0][l] = gw3;
+    red[w][1][l] = gb2;
+    red[w][2][l] = gb3;
   }
+  f32x16 acc, acch;
+#pragma unroll
+  for (int v = 0; v < 16; v++) acc[v] = acch[v] = 0.f;
   // ---- dW2[f][k] = sum_pt dZ2[f][pt] H1[pt][k]   (A = dZ2, B = H1 with K = points)
-  {
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int m = 0; m < 2; m++)
-#pragma unroll
-      for (int n2 = 0; n2 < 2; n2++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) acc[m][n2][v] = 0.f;
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-      bf16x8 a[2], b[2];
-#pragma unroll
-      for (int m = 0; m < 2; m++) a[m] = *(const bf16x8 *)(dz2 + (32 * m + lr) * kHStr + 16 * s + 8 * lh);
-#pragma unroll
-      for (int n2 = 0; n2 < 2; n2++) b[n2] = *(const bf16x8 *)(h1t + (32 * n2 + lr) * kHStr + 16 * s + 8 * lh);
-#pragma unroll
-      for (int m = 0; m < 2; m++)
-#pragma unroll
-        for (int n2 = 0; n2 < 2; n2++)
-          acc[m][n2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[m], b[n2], acc[m][n2], 0, 0, 0);
-    }
-#pragma unroll
-    for (int m = 0; m < 2; m++)
-#pragma unroll
-      for (int n2 = 0; n2 < 2; n2++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) g[kOffW2 + (32 * m + mfma_row(v, l)) * kMlpH + 32 * n2 + lr] = acc[m][n2][v];
-  }
-  __syncthreads();   // hs is rewritten below
   // ---- dH1^T[k][pt] = sum_f W2[f][k] dZ2[f][pt]   (A = W2^T, B = dZ2 with K = features)
-  {
-    f32x16 acc[2][2];
 #pragma unroll
-    for (int m = 0; m < 2; m++)
+  for (int s = 0; s < 4; s++) {
+    const bf16x8 a = *(const bf16x8 *)(dz2 + (32 * m + lr) * kHStr + 16 * s + 8 * lh);
+    const bf16x8 b = *(const bf16x8 *)(h1t + (32 * n2 + lr) * kHStr + 16 * s + 8 * lh);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+    const bf16x8 ah = *(const bf16x8 *)(M.w2t + (32 * m + lr) * kMlpH + 16 * s + 8 * lh);
+    const bf16x8 bh = *(const bf16x8 *)(dz2t + (32 * n2 + lr) * kHStr + 16 * s + 8 * lh);
+    acch = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, acch, 0, 0, 0);
+  }
 #pragma unroll
-      for (int n2 = 0; n2 < 2; n2++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) acc[m][n2][v] = 0.f;
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-      bf16x8 a[2], b[2];
-#pragma unroll
-      for (int m = 0; m < 2; m++) a[m] = *(const bf16x8 *)(M.w2t + (32 * m + lr) * kMlpH + 16 * s + 8 * lh);
-#pragma unroll
-      for (int n2 = 0; n2 < 2; n2++) b[n2] = *(const bf16x8 *)(dz2t + (32 * n2 + lr) * kHStr + 16 * s + 8 * lh);
-#pragma unroll
-      for (int m = 0; m < 2; m++)
-#pragma unroll
-        for (int n2 = 0; n2 < 2; n2++)
-          acc[m][n2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[m], b[n2], acc[m][n2], 0, 0, 0);
-    }
+  for (int v = 0; v < 16; v++) {
+    g[kOffW2 + (32 * m + mfma_row(v, l)) * kMlpH + 32 * n2 + lr] = acc[v];
     // dZ1 = relu'(z1) * dH1, with the forward pass's mask (h1 > 0)
-#pragma unroll
-    for (int m = 0; m < 2; m++)
-#pragma unroll
-      for (int n2 = 0; n2 < 2; n2++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-          const int k = 32 * m + mfma_row(v, l), pt = 32 * n2 + lr;
-          const bool on = (float)h1[pt * kHStr + k] > 0.f;
-          hs[k * (kWave + 1) + pt] = on ? acc[m][n2][v] : 0.f;
-        }
+    const int k = 32 * m + mfma_row(v, l), pt = 32 * n2 + lr;
+    const bool on = (float)h1[pt * kHStr + k] > 0.f;
+    dz1[k * (kWave + 1) + pt] = on ? acch[v] : 0.f;
   }
   __syncthreads();
   {
-    // lane k: dW1[k][0..2], db1[k]
-    const int k = l;
+    // lane k, points 16 w ..: dW1[k][0..2], db1[k]
     float gw[3] = {0.f, 0.f, 0.f}, gb = 0.f;
-    for (int pt = 0; pt < kWave; pt++) {
-      const float d = hs[k * (kWave + 1) + pt];
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      const int pt = 16 * w + e;
+      const float d = dz1[l * (kWave + 1) + pt];
       gb += d;
       for (int j = 0; j < 3; j++) gw[j] = fmaf(d, xsh[3 * pt + j], gw[j]);
     }
-    for (int j = 0; j < 3; j++) g[kOffW1 + 3 * k + j] = gw[j];
-    g[kOffB1 + k] = gb;
+    for (int j = 0; j < 3; j++) red[w][3 + j][l] = gw[j];
+    red[w][6][l] = gb;
+  }
+  __syncthreads();
+  // the waves' sums, in wave order
+  for (int i = threadIdx.x; i < 7 * kMlpH; i += kWave * kTrainWaves) {
+    const int what = i / kMlpH, k = i % kMlpH;
+    const float v = ((red[0][what][k] + red[1][what][k]) + red[2][what][k]) + red[3][what][k];
+    if (what == 0) g[kOffW3 + k] = v;
+    else if (what == 1) g[kOffB2 + k] = v;
+    else if (what == 2) {
+      if (k == 0) g[kOffB3] = v;
+    } else if (what < 6) g[kOffW1 + 3 * k + (what - 3)] = v;
+    else g[kOffB1 + k] = v;
   }
 }
 
-// gradient reduction in block order, Adam on the masters (skipped when
-// lr == 0), bf16 working copies
-__global__ void mlp_update_kernel(float *__restrict__ p, float *__restrict__ mom, float *__restrict__ vel,
-                                  float *__restrict__ wq, __bf16 *__restrict__ w2, __bf16 *__restrict__ w2t,
-                                  const float *__restrict__ part, int nblk, float *__restrict__ grad, float lr,
-                                  float beta1, float beta2, float eps, float bc1, float bc2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= kMlpNParam) return;
+// Gradient reduction in a fixed order, Adam on the masters (skipped when lr ==
+// 0), bf16 working copies.  A block takes kUpdP parameters and sums each one's
+// block partials in kUpdS slices (partials s, s + kUpdS, ...), then the slices
+// in order: with one thread per parameter, its 64 partials were a chain of
+// loads in 18 blocks (16.3 us, now 4.4).
+constexpr int kUpdP = 32, kUpdS = 16;
+__global__ void __launch_bounds__(kUpdP *kUpdS)
+    mlp_update_kernel(float *__restrict__ p, float *__restrict__ mom, float *__restrict__ vel, float *__restrict__ wq,
+                      __bf16 *__restrict__ w2, __bf16 *__restrict__ w2t, const float *__restrict__ part, int nblk,
+                      float *__restrict__ grad, float lr, float beta1, float beta2, float eps, float bc1, float bc2) {
+  __shared__ float sums[kUpdS][kUpdP];
+  const int i = blockIdx.x * kUpdP + threadIdx.x % kUpdP, sl = threadIdx.x / kUpdP;
+  float gs = 0.f;
+  if (i < kMlpNParam) {
+#pragma unroll 4
+    for (int b = sl; b < nblk; b += kUpdS) gs += part[(long)b * kMlpNParam + i];
+  }
+  sums[sl][threadIdx.x % kUpdP] = gs;
+  __syncthreads();
+  if (sl != 0 || i >= kMlpNParam) return;
   if (nblk > 0) {
-    float gs = 0.f;
-    for (int b = 0; b < nblk; b++) gs += part[(long)b * kMlpNParam + i];
+#pragma unroll
+    for (int s = 1; s < kUpdS; s++) gs += sums[s][threadIdx.x];
     if (grad) grad[i] = gs;
     if (lr > 0.f) {
       const float m1 = beta1 * mom[i] + (1.f - beta1) * gs;
@@ -268,7 +290,7 @@ int ensure_part(bamhip_mlp *m, long nblk) {
 }
 
 int refresh(bamhip_mlp *m) {
-  mlp_update_kernel<<<(kMlpNParam + 255) / 256, 256, 0, stream()>>>(m->p, m->mom, m->vel, m->wq, m->w2, m->w2t,
+  mlp_update_kernel<<<(kMlpNParam + kUpdP - 1) / kUpdP, kUpdP * kUpdS, 0, stream()>>>(m->p, m->mom, m->vel, m->wq, m->w2, m->w2t,
                                                                     nullptr, 0, nullptr, 0.f, 0.f, 0.f, 0.f, 1.f,
                                                                     1.f);
   BH_HIP(hipGetLastError());
@@ -280,14 +302,14 @@ int train_step(bamhip_mlp *m, const float *feat, const float *target, long n, lo
                unsigned long long pa, unsigned long long pb, float lr, float *grad_out) {
   const long nblk = (batch + kWave - 1) / kWave;
   if (int e = ensure_part(m, nblk)) return e;
-  mlp_train_kernel<<<(unsigned)nblk, kWave, 0, stream()>>>(mlp_view(m), feat, target, n, q0, batch, pa, pb, m->part,
+  mlp_train_kernel<<<(unsigned)nblk, kWave * kTrainWaves, 0, stream()>>>(mlp_view(m), feat, target, n, q0, batch, pa, pb, m->part,
                                                            m->lossp, 1.f / (float)batch);
   BH_HIP(hipGetLastError());
   const float b1 = 0.9f, b2 = 0.999f;
   if (lr > 0.f) m->step++;
   const float bc1 = 1.f - powf(b1, (float)std::max<long>(m->step, 1));
   const float bc2 = 1.f - powf(b2, (float)std::max<long>(m->step, 1));
-  mlp_update_kernel<<<(kMlpNParam + 255) / 256, 256, 0, stream()>>>(m->p, m->mom, m->vel, m->wq, m->w2, m->w2t,
+  mlp_update_kernel<<<(kMlpNParam + kUpdP - 1) / kUpdP, kUpdP * kUpdS, 0, stream()>>>(m->p, m->mom, m->vel, m->wq, m->w2, m->w2t,
                                                                     m->part, (int)nblk, grad_out, lr, b1, b2,
                                                                     1e-8f, bc1, bc2);
   BH_HIP(hipGetLastError());

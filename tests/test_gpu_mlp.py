@@ -206,3 +206,26 @@ def test_learned_hybrid_matches_reference_hybrid():
     # learned start converges on all but a few percent of the points (the
     # slowest-converging states of the distribution need more than 8)
     assert nfb - (st == O.C2P_NR).sum() <= 0.05 * n, (nfb, (st == O.C2P_NR).sum())
+
+
+@pytest.mark.parametrize("n", [1, 15, 63, 64, 65, 1000, 4097])
+def test_gradient_of_partial_blocks_matches_oracle(data, n):
+    """sample counts around the 64-sample blocks, their 16-sample quarters and
+    the 16 slices of the reduction.  The device sums n FP32 terms in blocks; a
+    term is rounded at 2^-24 and its bf16 factors, the same on both sides, may
+    round the other way where the FP32 value before them differs in its last bit
+    (2^-8 of one sample's term)."""
+    net = B.Mlp(seed=4)
+    p = _random_params(9)
+    nrm = _norm(data["feat"], data["tgt"])
+    net.set(p, nrm)
+    f, t = data["feat"].get()[:n], data["tgt"].get()[:n]
+    df, dt = B.DeviceArray.from_host(f), B.DeviceArray.from_host(t)
+    g, loss = net.grad(df, dt)
+    x, tt = M.inputs(nrm, f, t)
+    want_l, want = M.loss_and_grad(p.astype(np.float64), x, tt, emulate=True)
+    assert abs(loss - want_l) <= 1e-4 * want_l
+    assert np.linalg.norm(g - want) <= 2.0 ** -8 * np.linalg.norm(want)
+    for a in (df, dt):
+        a.free()
+    net.free()
