@@ -84,6 +84,13 @@ struct TimerScope {
 
 // collect the 25 device pointers of an index list (returns error if missing)
 int gather_ptrs(bamhip_level *lev, const int *idx, int n, double **out, const char *what);
+// whether no address is in the list twice
+inline bool distinct(double *const *p, int n) {
+  for (int a = 0; a < n; a++)
+    for (int b = 0; b < a; b++)
+      if (p[a] == p[b]) return false;
+  return true;
+}
 // looks up the device address of the fixed reduction scratch of output.hip
 // on `device` (current); called once per device by bamhip_init
 int noalloc_scratch_init(int device);

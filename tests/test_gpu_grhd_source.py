@@ -84,3 +84,43 @@ def test_sources_bitwise(eos, c, order):
     np.testing.assert_array_equal(got_madm, want_madm)
     rhs0c = np.concatenate([r.reshape(5, -1) for r in rhs0], axis=1)
     assert np.abs(got_rhs[2:] - rhs0c[2:]).max() > 1e-6      # momentum sources act
+
+
+def _one_box(shape, rhs_of, seed=7, c=0.125):
+    """The sources on one box with the rhs list rhs_of, on the device and from the oracle."""
+    m, n, o = shape
+    ob, gb = O.make_box(m, n, o, -1.0, -0.6, -0.5, H), B.make_box(m, n, o, -1.0, -0.6, -0.5, H, bflag=(B.PHYBOUND,) * 6)
+    met, K, prim = _fields(ob, seed)
+    rhs = np.random.default_rng(seed + 1).standard_normal((5, o, n, m))
+    lev = B.Level([gb], NV)
+    lev.enable(range(NV))
+    for vs, data in ((MET, met), (KIJ, K), (PRIM, prim), (RHS, rhs)):
+        for v, d in zip(vs, data):
+            lev.put(v, d.reshape(-1))
+    for v in MADM:
+        lev.fill(v, 0.0)
+    lev.grhd_sources(B.hrsc_params(eos="ideal"), rhs_of, MET, KIJ, PRIM, MADM, c=c, rhoatm=7e-4)
+    got = np.stack([lev.get(v) for v in RHS]), np.stack([lev.get(v) for v in MADM])
+    lev.free()
+    madm, add = np.zeros((11, o, n, m)), np.zeros((5, o, n, m))
+    want = rhs.copy()
+    O.grhd_sources(ob, O.hrsc_params(eos=0), met, K, prim, want, madm, c=c, rhoatm=7e-4)
+    O.grhd_sources(ob, O.hrsc_params(eos=0), met, K, prim, add, madm, c=c, rhoatm=7e-4)
+    return got, want.reshape(5, -1), madm.reshape(11, -1), rhs.reshape(5, -1), add.reshape(5, -1)
+
+
+@pytest.mark.parametrize("shape", [(7, 7, 7), (16, 4, 16), (17, 5, 17), (15, 16, 8), (33, 21, 9), (16, 37, 12)])
+def test_sources_at_tile_edges_bitwise(shape):
+    """Boxes at the edges of the 16x4x4 tiles and of the groups of four tile rows: bitwise the oracle's."""
+    (rhs, madm), want, wmadm, _, _ = _one_box(shape, RHS)
+    np.testing.assert_array_equal(rhs, want)
+    np.testing.assert_array_equal(madm, wmadm)
+
+
+def test_sources_into_one_variable_twice():
+    """A list that names a variable twice adds both sources to it, in the order of the list."""
+    (rhs, _), _, _, rhs0, add = _one_box((18, 9, 10), [0, 1, 2, 3, 2])
+    want = rhs0.copy()
+    for k, v in enumerate([0, 1, 2, 3, 2]):
+        want[v] = want[v] + add[k]
+    np.testing.assert_array_equal(rhs, want)
