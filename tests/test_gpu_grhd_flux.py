@@ -91,3 +91,39 @@ def test_fluxes_polytrope():
     scale = np.abs(want - rhs0).max()
     assert np.abs(got - want).max() <= 1e-12 * scale
     np.testing.assert_array_equal(got[1], rhs0[1])  # cold EOS: no tau flux
+
+
+def _one_box(shape, rhs_of, c=0.0625, seed=9):
+    ob, gb = O.make_box(*shape, -1.0, -1.0, -1.0, H), B.make_box(*shape, -1.0, -1.0, -1.0, H)
+    met, prim = _state(ob, seed)
+    rhs0 = np.random.default_rng(seed + 1).standard_normal((5, ob.o, ob.n, ob.m))
+    lev = B.Level([gb], NV)
+    lev.enable(range(NV))
+    for vs, data in ((MET, met), (PRIM, prim), (RHS, rhs0)):
+        for v, d in zip(vs, data):
+            lev.put(v, d.reshape(-1))
+    lev.grhd_fluxes(B.hrsc_params(eos="ideal", riemann="HLL", rec="WENOZ"), rhs_of, MET, PRIM, c=c)
+    got = np.stack([lev.get(v) for v in RHS])
+    lev.free()
+    op = O.hrsc_params(eos=0, riemann="HLL", rec="WENOZ")
+    want = O.grhd_fluxes(ob, op, met, prim, rhs0.copy(), c=c).reshape(5, -1)
+    add = O.grhd_fluxes(ob, op, met, prim, np.zeros_like(rhs0), c=c).reshape(5, -1)
+    return got, want, rhs0.reshape(5, -1), add
+
+
+@pytest.mark.parametrize("shape", [(62, 14, 17), (63, 15, 15), (64, 16, 16), (127, 5, 31), (16, 31, 4)])
+def test_fluxes_at_tile_edges_bitwise(shape):
+    """Lines that end just before, at and after the end of a tile of 63 (x) or 15 (y, z) points."""
+    got, want, _, _ = _one_box(shape, RHS)
+    np.testing.assert_array_equal(got, want)
+
+
+def test_fluxes_into_one_variable_twice():
+    """A list that names a variable twice takes both divergences: six sums, each rounded once."""
+    got, _, rhs0, add = _one_box((20, 18, 17), [0, 1, 2, 3, 0])
+    want = rhs0.copy()
+    want[0] = want[0] + add[0] + add[4]
+    want[1:4] = want[1:4] + add[1:4]
+    bound = 6 * np.finfo(float).eps * (np.abs(rhs0) + np.abs(add)).max() * 2
+    assert np.abs(got[4] - rhs0[4]).max() == 0.
+    assert np.abs(got[:4] - want[:4]).max() <= bound
