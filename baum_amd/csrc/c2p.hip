@@ -414,20 +414,32 @@ __device__ int c2p_bracketed_pt(const C2PK &P, double conD, double conS2, double
   return C2P_OK;
 }
 
+// conserved variables and metric of a point
+struct ConsIn {
+  double c[5], g[6];
+};
+__device__ __forceinline__ ConsIn load_cons(const C2PArrays &A, long q) {
+  ConsIn in;
+#pragma unroll
+  for (int k = 0; k < 6; k++) in.g[k] = A.g[k][q];
+#pragma unroll
+  for (int k = 0; k < 5; k++) in.c[k] = A.cons[k][q];
+  return in;
+}
+
 // undensitise and raise S with the inverse metric: shared by the bracketed
 // and learned solvers
 struct Undens {
   double D, T, S2, Six, Siy, Siz, detg;
 };
-__device__ __forceinline__ Undens undensitise(const C2PArrays &A, long q) {
+__device__ __forceinline__ Undens undensitise(const ConsIn &in) {
   Undens u;
   double gixx, gixy, gixz, giyy, giyz, gizz;
-  u.detg = invg(A.g[0][q], A.g[1][q], A.g[2][q], A.g[3][q], A.g[4][q], A.g[5][q], &gixx, &gixy, &gixz, &giyy,
-                &giyz, &gizz);
+  u.detg = invg(in.g[0], in.g[1], in.g[2], in.g[3], in.g[4], in.g[5], &gixx, &gixy, &gixz, &giyy, &giyz, &gizz);
   const double oo = 1. / sqrt(u.detg);
-  u.D = A.cons[0][q] * oo;
-  u.T = A.cons[1][q] * oo;
-  const double Sx = A.cons[2][q] * oo, Sy = A.cons[3][q] * oo, Sz = A.cons[4][q] * oo;
+  u.D = in.c[0] * oo;
+  u.T = in.c[1] * oo;
+  const double Sx = in.c[2] * oo, Sy = in.c[3] * oo, Sz = in.c[4] * oo;
   u.Six = gixx * Sx + gixy * Sy + gixz * Sz;
   u.Siy = gixy * Sx + giyy * Sy + giyz * Sz;
   u.Siz = gixz * Sx + giyz * Sy + gizz * Sz;
@@ -435,8 +447,8 @@ __device__ __forceinline__ Undens undensitise(const C2PArrays &A, long q) {
   return u;
 }
 
-__device__ __forceinline__ void store_prims(const C2PArrays &A, long q, const Undens &u, double rho, double eps,
-                                            double p) {
+__device__ __forceinline__ void store_prims(const C2PArrays &A, long q, const Undens &u, const double g[6], double rho,
+                                            double eps, double p) {
   const double ooDpT = 1.0 / (u.D + p + u.T);
   const double vx = u.Six * ooDpT, vy = u.Siy * ooDpT, vz = u.Siz * ooDpT;
   A.prim[0][q] = rho;
@@ -445,20 +457,22 @@ __device__ __forceinline__ void store_prims(const C2PArrays &A, long q, const Un
   A.prim[3][q] = vy;
   A.prim[4][q] = vz;
   A.prim[5][q] = p;
-  const double vlx = A.g[0][q] * vx + A.g[1][q] * vy + A.g[2][q] * vz;
-  const double vly = A.g[1][q] * vx + A.g[3][q] * vy + A.g[4][q] * vz;
-  const double vlz = A.g[2][q] * vx + A.g[4][q] * vy + A.g[5][q] * vz;
+  const double vlx = g[0] * vx + g[1] * vy + g[2] * vz;
+  const double vly = g[1] * vx + g[3] * vy + g[4] * vz;
+  const double vlz = g[2] * vx + g[4] * vy + g[5] * vz;
   A.prim[6][q] = vlx * vx + vly * vy + vlz * vz;
   A.prim[7][q] = u.detg;
 }
 
 __global__ void c2p_bracketed_kernel(C2PArrays A, C2PK P, long n) {
   for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
-    const Undens u = undensitise(A, q);
+    const Undens u = undensitise(load_cons(A, q));
     double rho, eps, p;
     int it;
     const int st = c2p_bracketed_pt(P, u.D, u.S2, u.T, A.prim[5][q], &rho, &eps, &p, &it, P.countmax);
-    store_prims(A, q, u, rho, eps, p);
+    double g[6];  // read again rather than kept over the solve, before the stores
+    for (int k = 0; k < 6; k++) g[k] = A.g[k][q];
+    store_prims(A, q, u, g, rho, eps, p);
     A.status[q] = st;
     A.iters[q] = it;
   }
@@ -501,36 +515,35 @@ __global__ void c2p_bracketed_hybrid_kernel(C2PArrays A, C2PK P, long n) {
 // predicted pressure, limited to polish_max iterations.  A point whose
 // features are not finite or whose polish does not converge falls back to
 // the cold-started bracketed solve (counted in *fallbacks).  The loop trip
-// count is uniform over the block, so every wave reaches the barriers.
+// count is uniform over the block, so every lane takes part in the network.
+// 4M points: 325 us with the activations through LDS and every load at its use;
+// 315 us with the activations in registers, 296 us with the next tile's inputs
+// loaded before the solve and the metric kept for the end (161 us of traffic).
+// Two waves per SIMD (229 registers): at three the network goes half the points
+// at a time, reads its weights twice, and takes 369 us.
 __global__ void __launch_bounds__(64) c2p_learned_kernel(C2PArrays A, C2PK P, MlpView M, long n, int polish_max,
                                                          int *fallbacks) {
-  // one wavefront per block: the barriers only order this wave's LDS traffic
-  __shared__ __attribute__((aligned(16))) __bf16 h1[64 * kHStr];
-  __shared__ __attribute__((aligned(16))) float b2[kMlpH], w3[kMlpH], w1b1[4 * kMlpH];
+  __shared__ __attribute__((aligned(16))) float b2[kMlpH], w3[kMlpH];
+  __shared__ float4 w1[kMlpH];
   const int l = threadIdx.x;
   b2[l] = M.p[kOffB2 + l];
   w3[l] = M.wq[192 + l];
-  for (int j = 0; j < 3; j++) w1b1[3 * l + j] = M.wq[3 * l + j];
-  w1b1[192 + l] = M.p[kOffB1 + l];
+  w1[l] = make_float4(M.wq[3 * l], M.wq[3 * l + 1], M.wq[3 * l + 2], M.p[kOffB1 + l]);
   __syncthreads();
   int nfb = 0;
-  for (long base = (long)blockIdx.x * 64; base < n; base += (long)gridDim.x * 64) {
+  const long step = (long)gridDim.x * 64;
+  ConsIn in = load_cons(A, min((long)blockIdx.x * 64 + l, n - 1));
+  for (long base = (long)blockIdx.x * 64; base < n; base += step) {
     const long q = base + l;
     const bool act = q < n;
-    Undens u = {};
-    double th = 0.;
-    float x[3] = {0.f, 0.f, 0.f};
-    bool valid = false;
-    if (act) {
-      u = undensitise(A, q);
-      th = mlp_thermal(u.D, u.S2, u.T);
-      valid = mlp_features(M, u.D, u.S2, u.T, th, x);
-      if (!valid) x[0] = x[1] = x[2] = 0.f;
-    }
-    mlp_layer1_from(w1b1, x, h1 + l * kHStr);
-    __syncthreads();
-    const float yn = mlp_infer23(M, h1, b2, w3);
-    __syncthreads();
+    const Undens u = undensitise(in);
+    const double g[6] = {in.g[0], in.g[1], in.g[2], in.g[3], in.g[4], in.g[5]};
+    const double th = mlp_thermal(u.D, u.S2, u.T);
+    float x[3];
+    const bool valid = mlp_features(M, u.D, u.S2, u.T, th, x);
+    if (!valid) x[0] = x[1] = x[2] = 0.f;
+    const float yn = mlp_infer(M, x, w1, b2, w3);
+    in = load_cons(A, min(q + step, n - 1));  // the next tile's, while this one is solved and stored
     if (act) {
       double rho = 0., eps = 0., p = 0.;
       int it = 0, it2 = 0, st = C2P_NR;
@@ -542,7 +555,7 @@ __global__ void __launch_bounds__(64) c2p_learned_kernel(C2PArrays A, C2PK P, Ml
         nfb++;
         st = c2p_bracketed_pt(P, u.D, u.S2, u.T, 0., &rho, &eps, &p, &it2, P.countmax);
       }
-      store_prims(A, q, u, rho, eps, p);
+      store_prims(A, q, u, g, rho, eps, p);
       A.status[q] = st;
       A.iters[q] = it + it2;
     }
@@ -561,16 +574,15 @@ __global__ void __launch_bounds__(64) c2p_learned_kernel(C2PArrays A, C2PK P, Ml
 // reference's rules.  A state with D < fatm rhoatm (rho = D / W is then
 // below the atmosphere threshold whatever the pressure) and a state with no
 // thermal content skip the network.  The loop trip count is uniform over
-// the block, so every wave reaches the barriers.
+// the block, so every lane takes part in the network.
 __global__ void __launch_bounds__(64) c2p_learned_hybrid_kernel(C2PArrays A, C2PK P, MlpView M, long n,
                                                                 int polish_max, int *fallbacks) {
-  __shared__ __attribute__((aligned(16))) __bf16 h1[64 * kHStr];
-  __shared__ __attribute__((aligned(16))) float b2[kMlpH], w3[kMlpH], w1b1[4 * kMlpH];
+  __shared__ __attribute__((aligned(16))) float b2[kMlpH], w3[kMlpH];
+  __shared__ float4 w1[kMlpH];
   const int l = threadIdx.x;
   b2[l] = M.p[kOffB2 + l];
   w3[l] = M.wq[192 + l];
-  for (int j = 0; j < 3; j++) w1b1[3 * l + j] = M.wq[3 * l + j];
-  w1b1[192 + l] = M.p[kOffB1 + l];
+  w1[l] = make_float4(M.wq[3 * l], M.wq[3 * l + 1], M.wq[3 * l + 2], M.p[kOffB1 + l]);
   __syncthreads();
   C2PK Pl = P;
   Pl.countmax = polish_max;
@@ -590,10 +602,7 @@ __global__ void __launch_bounds__(64) c2p_learned_hybrid_kernel(C2PArrays A, C2P
       }
       if (!valid) x[0] = x[1] = x[2] = 0.f;
     }
-    mlp_layer1_from(w1b1, x, h1 + l * kHStr);
-    __syncthreads();
-    const float yn = mlp_infer23(M, h1, b2, w3);
-    __syncthreads();
+    const float yn = mlp_infer(M, x, w1, b2, w3);
     if (act) {
       double rho = 0., epsl = 0., pres = 0.;
       int it = 0, result = h.result;
@@ -622,7 +631,7 @@ __global__ void __launch_bounds__(64) c2p_learned_hybrid_kernel(C2PArrays A, C2P
 // succeed or the state has no thermal content
 __global__ void mlp_prepare_kernel(C2PArrays A, C2PK P, long n, float *__restrict__ feat, float *__restrict__ target) {
   for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
-    const Undens u = undensitise(A, q);
+    const Undens u = undensitise(load_cons(A, q));
     const double th = mlp_thermal(u.D, u.S2, u.T);
     float r[3];
     const bool fok = mlp_raw_features(u.D, u.S2, u.T, th, r);
