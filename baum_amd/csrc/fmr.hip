@@ -63,14 +63,15 @@ struct RJob {
 };
 struct RArgs {
   int njobs;
+  unsigned nblk;  // blocks of all jobs
   RJob job[kMaxJobs];
   double c[8];
 };
 
 template <class J>
-__device__ __forceinline__ int find_job(const J *job, int njobs) {
+__device__ __forceinline__ int find_job(const J *job, int njobs, unsigned b) {
   int jb = 0;
-  while (jb + 1 < njobs && (long)blockIdx.x >= job[jb + 1].blk0) jb++;
+  while (jb + 1 < njobs && (long)b >= job[jb + 1].blk0) jb++;
   return jb;
 }
 
@@ -80,7 +81,7 @@ __device__ __forceinline__ int find_job(const J *job, int njobs) {
 // window shifted by one): interpolate_boxtobox_N.c:652-672, 712-731, 770-794.
 template <int N>
 __global__ void __launch_bounds__(kBlock) prolong_kernel(PArgs a, VarPtrs vp) {
-  const int jb = find_job(a.job, a.njobs);
+  const int jb = find_job(a.job, a.njobs, blockIdx.x);
   const PJob &J = a.job[jb];
   const long q = ((long)blockIdx.x - J.blk0) * kBlock + threadIdx.x;
   if (q >= J.noct) return;
@@ -179,7 +180,10 @@ __device__ __forceinline__ void stage_tile(double *t, const double *__restrict__
 // left child sums terms 0..N-1 of its window with c1, a right child terms
 // 1..N with c2, each from 0 in increasing order), so the results are bitwise
 // equal; the coarse data is read once per tile instead of (N+1)^3 / 8 times
-// per fine point.
+// per fine point.  Bound by LDS reads and latency: with one child per thread and
+// a branch on which, the wavefronts ran both sides and read every term twice
+// (96^3 fine points, 25 variables, order 4: 63 us); both children of a column
+// from one set of reads, and in x a thread that keeps its child, take 49 us.
 constexpr int PTX = 8, PTY = 4, PTZ = 4;
 template <int N>
 __global__ void __launch_bounds__(kBlock) prolong_tile_kernel(PArgs a, VarPtrs vp) {
@@ -187,7 +191,7 @@ __global__ void __launch_bounds__(kBlock) prolong_tile_kernel(PArgs a, VarPtrs v
   __shared__ double cin[CZ * CY * CX];
   __shared__ double dz[2 * PTZ * CY * CX];   // [fine z][coarse y][coarse x]
   __shared__ double dy[2 * PTZ * 2 * PTY * CX];  // [fine z][fine y][coarse x]
-  const int jb = find_job(a.job, a.njobs);
+  const int jb = find_job(a.job, a.njobs, blockIdx.x);
   const PJob &J = a.job[jb];
   const long b = (long)blockIdx.x - J.blk0;
   const int ox0 = (int)(b % J.ntx) * PTX, oy0 = (int)((b / J.ntx) % J.nty) * PTY,
@@ -214,54 +218,54 @@ __global__ void __launch_bounds__(kBlock) prolong_tile_kernel(PArgs a, VarPtrs v
   const int ex = vx + N, ey = vy + N, ez = vz + N;  // coarse points the valid octets read
   stage_tile<CX, CY, CZ>(cin, cv, J.cm, J.cmn, ex, ey, ez, tid);
   __syncthreads();
-  for (int idx = tid; idx < 2 * PTZ * CY * CX; idx += kBlock) {  // z sums
-    const int x = idx % CX, y = (idx / CX) % CY, fz = idx / (CX * CY);
-    const int oz = fz / 2, sz = fz % 2;
-    double d = 0;
-    if (sz == 0) {
+  // z sums, both children of a column per thread
+  for (int idx = tid; idx < PTZ * CY * CX; idx += kBlock) {
+    const int xy = idx % (CX * CY), oz = idx / (CX * CY);
+    double u[N + 1], d0 = 0, d1 = 0;
 #pragma unroll
-      for (int p = 0; p < N; p++) d += a.c1[p] * cin[x + CX * (y + CY * (oz + p))];
-    } else {
+    for (int p = 0; p <= N; p++) u[p] = cin[xy + CX * CY * (oz + p)];
 #pragma unroll
-      for (int p = 0; p < N; p++) d += a.c2[p] * cin[x + CX * (y + CY * (oz + p + 1))];
-    }
-    dz[idx] = d;
+    for (int p = 0; p < N; p++) d0 += a.c1[p] * u[p];
+#pragma unroll
+    for (int p = 0; p < N; p++) d1 += a.c2[p] * u[p + 1];
+    dz[xy + CX * CY * (2 * oz)] = d0;
+    dz[xy + CX * CY * (2 * oz + 1)] = d1;
   }
   __syncthreads();
-  for (int idx = tid; idx < 4 * PTZ * PTY * CX; idx += kBlock) {  // y sums
-    const int x = idx % CX, fy = (idx / CX) % (2 * PTY), fz = idx / (CX * 2 * PTY);
-    const int oy = fy / 2, r = fy % 2;
-    double e = 0;
-    if (r == 0) {
+  // y sums, likewise
+  for (int idx = tid; idx < 2 * PTZ * PTY * CX; idx += kBlock) {
+    const int x = idx % CX, oy = (idx / CX) % PTY, fz = idx / (CX * PTY);
+    double u[N + 1], e0 = 0, e1 = 0;
 #pragma unroll
-      for (int by = 0; by < N; by++) e += a.c1[by] * dz[x + CX * ((oy + by) + CY * fz)];
-    } else {
+    for (int by = 0; by <= N; by++) u[by] = dz[x + CX * ((oy + by) + CY * fz)];
 #pragma unroll
-      for (int by = 1; by <= N; by++) e += a.c2[by - 1] * dz[x + CX * ((oy + by) + CY * fz)];
-    }
-    dy[idx] = e;
+    for (int by = 0; by < N; by++) e0 += a.c1[by] * u[by];
+#pragma unroll
+    for (int by = 0; by < N; by++) e1 += a.c2[by] * u[by + 1];
+    dy[x + CX * (2 * oy + 2 * PTY * fz)] = e0;
+    dy[x + CX * (2 * oy + 1 + 2 * PTY * fz)] = e1;
   }
   __syncthreads();
-  double *__restrict__ fv = vp.dst[v] + J.foff;
-  for (int idx = tid; idx < 8 * PTX * PTY * PTZ; idx += kBlock) {  // x sums and stores
-    const int fx = idx % (2 * PTX), fy = (idx / (2 * PTX)) % (2 * PTY), fz = idx / (4 * PTX * PTY);
-    const int ox = fx / 2, oy = fy / 2, oz = fz / 2, ac = fx % 2;
-    if (ox >= vx || oy >= vy || oz >= vz) continue;
-    const int fi = J.ifb[0] + 2 * (ox0 + ox), j = J.ifb[2] + 2 * oy0 + fy, k = J.ifb[4] + 2 * oz0 + fz;
-    const bool valid = j <= J.ifb[3] && k <= J.ifb[5];
-    const bool skip = fi >= J.ifb0[0] && fi <= J.ifb0[1] && j >= J.ifb0[2] && j <= J.ifb0[3] && k >= J.ifb0[4] &&
-                      k <= J.ifb0[5];
-    if (!valid || skip) continue;
-    const double *row = dy + CX * (fy + 2 * PTY * fz);
+  // x sums and stores, one fine point per thread (consecutive lanes store
+  // consecutive points); a thread keeps its fx and fy, and so its child
+  static_assert(kBlock % (4 * PTX * PTY) == 0, "a thread's fine x and y are the same in every pass");
+  const int fx = tid % (2 * PTX), fy = (tid / (2 * PTX)) % (2 * PTY);
+  const int ox = fx / 2, ac = fx % 2;
+  const int fi = J.ifb[0] + 2 * (ox0 + ox), j = J.ifb[2] + 2 * oy0 + fy;
+  if (ox >= vx || fy / 2 >= vy || j > J.ifb[3]) return;
+  const bool inxy = fi >= J.ifb0[0] && fi <= J.ifb0[1] && j >= J.ifb0[2] && j <= J.ifb0[3];
+  double c[N];
+#pragma unroll
+  for (int p = 0; p < N; p++) c[p] = ac == 0 ? a.c1[p] : a.c2[p];
+  double *__restrict__ fv = vp.dst[v] + J.foff + fi + ac + (long)j * J.fm;
+  for (int fz = tid / (4 * PTX * PTY); fz < 2 * PTZ; fz += kBlock / (4 * PTX * PTY)) {
+    const int k = J.ifb[4] + 2 * oz0 + fz;
+    if (fz / 2 >= vz || k > J.ifb[5] || (inxy && k >= J.ifb0[4] && k <= J.ifb0[5])) continue;
+    const double *row = dy + CX * (fy + 2 * PTY * fz) + ox + ac;
     double o = 0;
-    if (ac == 0) {
 #pragma unroll
-      for (int ax = 0; ax < N; ax++) o += a.c1[ax] * row[ox + ax];
-    } else {
-#pragma unroll
-      for (int ax = 1; ax <= N; ax++) o += a.c2[ax - 1] * row[ox + ax];
-    }
-    fv[fi + ac + (long)j * J.fm + (long)k * J.fmn] = o;
+    for (int p = 0; p < N; p++) o += c[p] * row[p];
+    fv[(long)k * J.fmn] = o;
   }
 }
 
@@ -270,7 +274,7 @@ __global__ void __launch_bounds__(kBlock) prolong_tile_kernel(PArgs a, VarPtrs v
 // accumulated in the reference's order.
 template <int N>
 __global__ void __launch_bounds__(kBlock) restrict_kernel(RArgs a, VarPtrs vp) {
-  const int jb = find_job(a.job, a.njobs);
+  const int jb = find_job(a.job, a.njobs, blockIdx.x);
   const RJob &J = a.job[jb];
   const long q = ((long)blockIdx.x - J.blk0) * kBlock + threadIdx.x;
   if (q >= J.npts) return;
@@ -303,7 +307,12 @@ __global__ void __launch_bounds__(kBlock) restrict_kernel(RArgs a, VarPtrs vp) {
 // sums as in restrict_kernel (a z sum e(ax, by) per fine column, then
 // dv(ax) = 0 + c0 e(ax, 0) + ..., then 0 + c0 dv(0) + ...), so the results
 // are bitwise equal; the fine data is read from HBM once instead of N^3 / 8
-// times.
+// times.  Order 4 stages 1.6 times the fine points: with neighbouring tiles on
+// different XCDs the common ones came from memory each time (96^3 fine points,
+// 25 variables: 59 us alone, 40 us in a hierarchy's steps); as runs of tiles per
+// XCD they come from its L2 (51 and 34 us).  Prolongation is not numbered so: its
+// tiles inside the skipped box are empty, and the XCDs with the middle of the box
+// would have less to do (49 -> 58 us).
 constexpr int RTX = 8, RTY = 8, RTZ = 4;
 template <int N>
 __global__ void __launch_bounds__(kBlock) restrict_tile_kernel(RArgs a, VarPtrs vp) {
@@ -311,9 +320,13 @@ __global__ void __launch_bounds__(kBlock) restrict_tile_kernel(RArgs a, VarPtrs 
   __shared__ double fin[FZ * FY * FX];
   __shared__ double ez[RTZ * FY * FX];
   __shared__ double ey[RTZ * RTY * FX];
-  const int jb = find_job(a.job, a.njobs);
+  // workgroup w runs on XCD w mod 8 (the grid is padded to a multiple of 8), and
+  // each XCD takes one run of tiles
+  const unsigned t = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;
+  if (t >= a.nblk) return;
+  const int jb = find_job(a.job, a.njobs, t);
   const RJob &J = a.job[jb];
-  const long b = (long)blockIdx.x - J.blk0;
+  const long b = (long)t - J.blk0;
   const int tx0 = (int)(b % J.ntx) * RTX, ty0 = (int)((b / J.ntx) % J.nty) * RTY,
             tz0 = (int)(b / ((long)J.ntx * J.nty)) * RTZ;
   const int vx = min(RTX, J.ncx - tx0), vy = min(RTY, J.ncy - ty0), vz = min(RTZ, J.ncz - tz0);
@@ -604,6 +617,7 @@ int launch_restrict(RArgs &args, const std::vector<RJob> &jobs, double *const *d
     args.njobs = nj;
     const long blk = assign_blocks(args.job, jobs.data() + j0, nj, g_restrict_lds ? restrict_tiles : restrict_units);
     if (blk == 0) continue;
+    args.nblk = (unsigned)blk;
     for (int v0 = 0; v0 < n; v0 += kMaxVars) {
       const int nv = std::min(kMaxVars, n - v0);
       VarPtrs vp{};
@@ -611,7 +625,7 @@ int launch_restrict(RArgs &args, const std::vector<RJob> &jobs, double *const *d
         vp.dst[v] = dst[v0 + v];
         vp.src[v] = src[v0 + v];
       }
-      const dim3 grid((unsigned)blk, (unsigned)nv);
+      const dim3 grid((unsigned)(g_restrict_lds ? (blk + 7) / 8 * 8 : blk), (unsigned)nv);
       hipStream_t st = stream();
       if (g_restrict_lds) {
         switch (order) {

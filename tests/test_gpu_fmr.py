@@ -193,3 +193,33 @@ def test_rejects_bad_calls():
     B.set_rp_flags(lc2, lf2, [0], 6, FP, FR)
     with pytest.raises(B.BamhipError, match="too small"):
         B.prolong_varlist(lc2, lf2, [U0], [U0], order=4)
+
+
+@pytest.mark.parametrize("order", [2, 4, 8])
+@pytest.mark.parametrize("size", [(48, 48, 24), (50, 46, 26), (66, 34, 44)])
+def test_coupling_of_many_tiles_matches_oracle_bitwise(size, order):
+    """one box of several tiles in each direction (whole ones, one point more, one less): tiles with
+    neighbours on all sides, tiles inside the skipped box and numbers of tiles that 8 does not divide"""
+    nb, nvar = 6, 2
+    both = []
+    for mk in (_mk, _omk):
+        cb = coarse_box(mk, 44, 36, 34, 0.5)
+        both.append((cb, fine_box(mk, cb, (5, 6, 5), size)))
+    (cb, fb), (ocb, ofb) = both
+    lc, lf = B.Level([cb], U0 + nvar, l=0), B.Level([fb], U0 + nvar, l=1)
+    lc.enable(range(U0 + nvar))
+    lf.enable(range(U0 + nvar))
+    B.set_rp_flags(lc, lf, [0], nb, FP, FR)
+    cv, fv = _random_levels(lc, lf, nvar, 300 + order)
+    idx = list(range(U0, U0 + nvar))
+    fp, fr = O.rp_flags([ofb], [ocb], [0], nb)
+    wc, wf = cv.copy(), fv.copy()
+    assert O.restrict_level([ofb], [ocb], [0], fr, 3, order, fv, wc) == 0
+    assert O.prolong_level([ofb], [ocb], [0], fp, 3, nb, order, cv, wf) == 0
+    B.restrict_varlist(lf, lc, idx, idx, nbuffer=3, order=order)
+    np.testing.assert_array_equal(np.array([lc.get(v) for v in idx]), wc)
+    for v in range(nvar):
+        lc.put(U0 + v, cv[v])
+    B.prolong_varlist(lc, lf, idx, idx, nbuffer=3, order=order)
+    np.testing.assert_array_equal(np.array([lf.get(v) for v in idx]), wf)
+    assert np.count_nonzero(wc != cv) > 0 and np.count_nonzero(wf != fv) > 0
