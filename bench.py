@@ -70,7 +70,7 @@ def parse():
     ap.add_argument("--cpu-seconds", type=float, default=12.0, help="target CPU-baseline sample time")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--rhs-overlap", type=int, default=1,
-                    help="1: box-edge shell kernels concurrent with the bulk kernel (second stream)")
+                    help="1: box-edge shell tiles and bulk tiles in one launch; 0: one after the other")
     ap.add_argument("--rk-fusion", type=int, default=2,
                     help="RK4 stage update inside the RHS kernels: 0 never, 1 always, 2 on levels >= 2^19 points")
     ap.add_argument("--xcd-map", type=int, default=1, help="1: XCD-aware tile numbering in the RHS kernels")
@@ -780,7 +780,7 @@ def main():
                                       "frac": rate / PEAK_FP64_TFLOPS, "rhs_ms_per_coarse_step": rhs_ms,
                                       "flop_per_coarse_step": rhs_flop,
                                       "kernels": "every Z4c RHS launch of one eagerly run coarse step: bulk and "
-                                                 "shell tiles on two streams, RK4 update fused into the store"}
+                                                 "shell tiles in one launch, RK4 update fused into the store"}
     elif box:
         out.update(value=box["value"], unit="grid-point-updates/s", ms_per_step=box["ms_per_step"])
         out["config"] = {"workload": "Z4c RK4, one 192^3 periodic box", "parallelism": "single GPU"}
