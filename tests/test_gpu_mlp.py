@@ -229,3 +229,35 @@ def test_gradient_of_partial_blocks_matches_oracle(data, n):
     for a in (df, dt):
         a.free()
     net.free()
+
+
+def _learned(net, P, cons, g):
+    n = cons.shape[1]
+    arrays = dc, dg, dpr, ds, di, fb = (B.DeviceArray.from_host(np.ascontiguousarray(cons)),
+                                        B.DeviceArray.from_host(np.ascontiguousarray(g)),
+                                        B.DeviceArray.from_host(np.zeros((8, n))), B.DeviceArray((n,), np.int32),
+                                        B.DeviceArray((n,), np.int32), B.DeviceArray.from_host(np.zeros(1, np.int32)))
+    B.c2p_learned_batch(P, net, dc, dg, dpr, ds, di, fb, polish_max=8)
+    out = np.concatenate([dpr.get(), ds.get()[None], di.get()[None]]), int(fb.get()[0])
+    for a in arrays:
+        a.free()
+    return out
+
+
+@pytest.mark.parametrize("n", [1, 31, 63, 64, 65, 4095, (1 << 21) + 77])
+def test_learned_points_do_not_depend_on_their_batch(n):
+    """A point's primitives, status and iterations are its own, bitwise: in wavefronts with idle lanes, and
+    where a wavefront takes several tiles of 64 points (more than 2^21 points)."""
+    base = _solved(4096, seed=45)
+    net = B.Mlp(seed=4)
+    net.set(None, _norm(base["feat"], base["tgt"]))
+    cons, g = base["cons0"], base["g"].get()
+    cons[:, 7] = np.nan                     # no features: the fallback solve
+    want, fb = _learned(net, base["P"], cons, g)
+    k = np.arange(n) % 4096
+    got, _ = _learned(net, base["P"], cons[:, k], g[:, k])
+    np.testing.assert_array_equal(got, want[:, k])
+    assert fb >= 1
+    for a in (base["feat"], base["tgt"], base["g"]):
+        a.free()
+    net.free()
