@@ -68,7 +68,9 @@ struct RadInfo {
 // One thread per surface point of one box and variable (blockIdx.y).  The
 // kernel is bound by latency: a thread that looped over the 25 variables waited
 // for each one's neighbours in turn, 43 us on a 26^3 box and 59 us on a 66^3 box
-// whatever the number of points.
+// whatever the number of points.  CROSSED: an output is an operand or an output
+// of another variable, so one thread takes all variables of its point, reads
+// every operand before it stores, and stores in the order of the lists.
 // rk = 0: unew = RHS (c == 0) or upre + c RHS at the boundary points; rk = 1
 // (an RK4 stage with the update fused in): uc = ucin + wc RHS, when has_v
 // unew = upre + wv RHS, when has_cp copy = upre
@@ -77,6 +79,7 @@ struct RkFuse {
   double wc, wv;
   int rk, has_v, has_cp;
 };
+template <bool CROSSED>
 __global__ void radiative_kernel(Ptrs25 unew, Ptrs25 upre, Ptrs25 ucur, RadInfo ri, DevBox B, double c, RkFuse F) {
   const int M = B.m, N = B.n, O = B.o;
   const long nface_x = (long)N * O, nface_y = (long)(M - 2) * O, nface_z = (long)(M - 2) * (N - 2);
@@ -137,23 +140,36 @@ __global__ void radiative_kernel(Ptrs25 unew, Ptrs25 upre, Ptrs25 ucur, RadInfo 
     if (p != q && m != q) return cen;
     return (m == q) ? rgt : lft;
   };
-  {
-    const int v = blockIdx.y;
+  struct Point {
+    double rhs, a, b;
+  };
+  const auto load = [&](int v) {
     const double *u = ucur.p[v];
     const double sp = ri.v[v];
     const double vx = sp * nx, vy = sp * ny, vz = sp * nz;
-    double rhs = -sp * (u[q] - ri.var0[v]) / rr;
-    rhs -= vx * del(u, vx, Mcc, mcc, pcc, Pcc) / (2 * B.dx) + vy * del(u, vy, cMc, cmc, cpc, cPc) / (2 * B.dy) +
-           vz * del(u, vz, ccM, ccm, ccp, ccP) / (2 * B.dz);
+    Point w;
+    w.rhs = -sp * (u[q] - ri.var0[v]) / rr;
+    w.rhs -= vx * del(u, vx, Mcc, mcc, pcc, Pcc) / (2 * B.dx) + vy * del(u, vy, cMc, cmc, cpc, cPc) / (2 * B.dy) +
+             vz * del(u, vz, ccM, ccm, ccp, ccP) / (2 * B.dz);
+    w.a = F.rk ? F.ucin.p[v][q] : 0.0;
+    w.b = (F.rk ? F.has_v || F.has_cp : c != 0.0) ? upre.p[v][q] : 0.0;
+    return w;
+  };
+  const auto store = [&](int v, const Point &w) {
     if (F.rk) {
-      // both loads before the stores: an output may alias ucin or upre
-      const double a = F.ucin.p[v][q], b = (F.has_v || F.has_cp) ? upre.p[v][q] : 0.0;
-      F.uc.p[v][q] = a + F.wc * rhs;
-      if (F.has_v) unew.p[v][q] = b + F.wv * rhs;
-      if (F.has_cp) F.copy.p[v][q] = b;
+      F.uc.p[v][q] = w.a + F.wc * w.rhs;
+      if (F.has_v) unew.p[v][q] = w.b + F.wv * w.rhs;
+      if (F.has_cp) F.copy.p[v][q] = w.b;
     } else {
-      unew.p[v][q] = (c != 0.0) ? upre.p[v][q] + c * rhs : rhs;
+      unew.p[v][q] = (c != 0.0) ? w.b + c * w.rhs : w.rhs;
     }
+  };
+  if constexpr (CROSSED) {
+    Point w[25];
+    for (int v = 0; v < 25; v++) w[v] = load(v);
+    for (int v = 0; v < 25; v++) store(v, w[v]);
+  } else {
+    store(blockIdx.y, load(blockIdx.y));
   }
 }
 
@@ -645,6 +661,19 @@ static int boundary_impl(bamhip_level *lev, const bamhip_z4c_params *par, Ptrs25
     ri.var0[v] = (v == 0 || v == 3 || v == 5 || v == 6 || v == 18) ? 1.0 : 0.0;
     ri.v[v] = (v == 6 || v == 18 || v == 13) ? vg : 1.0;
   }
+  // variables run in blocks of their own: no order between an output and
+  // another variable's operands or outputs
+  const double *const *out[3] = {N.p, F.uc.p, F.copy.p}, *const *in[2] = {Pp.p, F.ucin.p};
+  const bool has_out[3] = {!F.rk || F.has_v, F.rk != 0, F.rk && F.has_cp},
+             has_in[2] = {F.rk ? F.has_v || F.has_cp : c != 0.0, F.rk != 0};
+  bool crossed = false;
+  for (int v = 0; v < 25; v++)
+    for (int w = 0; w < 25; w++)
+      for (int x = 0; x < 3; x++) {
+        if (v == w || !has_out[x]) continue;
+        for (int y = 0; y < 2; y++) crossed |= has_in[y] && out[x][v] == in[y][w];
+        for (int y = 0; y < 3; y++) crossed |= has_out[y] && out[x][v] == out[y][w];
+      }
   TimerScope t("set_boundary");
   for (const DevBox &B : lev->boxes) {
     bool anyphy = false, anyper = false;
@@ -655,7 +684,9 @@ static int boundary_impl(bamhip_level *lev, const bamhip_z4c_params *par, Ptrs25
     if (anyphy) {
       if (B.m < 3 || B.n < 3 || B.o < 3) return set_error(BAMHIP_EINVAL, "%s: box too small for the radiative condition", what);
       const long total = 2L * ((long)B.n * B.o + (long)(B.m - 2) * B.o + (long)(B.m - 2) * (B.n - 2));
-      radiative_kernel<<<dim3((unsigned)((total + 255) / 256), 25, 1), 256, 0, stream()>>>(N, Pp, U, ri, B, c, F);
+      const unsigned nblk = (unsigned)((total + 255) / 256);
+      if (crossed) radiative_kernel<true><<<nblk, 256, 0, stream()>>>(N, Pp, U, ri, B, c, F);
+      else radiative_kernel<false><<<dim3(nblk, 25, 1), 256, 0, stream()>>>(N, Pp, U, ri, B, c, F);
       BH_HIP(hipGetLastError());
     }
     if (anyper) {

@@ -149,3 +149,61 @@ def test_lists_crossed_between_fields():
     for x, y in zip(out[0][:2], out[1][:2]):
         scale = np.abs(x[:, on]).max(axis=1, keepdims=True)
         assert (np.abs(x - y)[:, on] <= 1e-12 * scale).all()
+
+
+def _bc_stage(lev, par, src, acc, accout, base, vout, copy, wc, wv):
+    L = B.lib()
+    ip = C.POINTER(C.c_int)
+    L.bamhip_z4c_bc_rk4_stage.restype = C.c_int
+    L.bamhip_z4c_bc_rk4_stage.argtypes = [C.c_void_p, C.POINTER(B.Z4cParams)] + [ip] * 6 + [C.c_double] * 2 + [C.c_int] * 2
+    arr = lambda x: None if x is None else (C.c_int * 25)(*x)  # noqa: E731
+    B.check(L.bamhip_z4c_bc_rk4_stage(lev.h, C.byref(par), arr(src), arr(acc), arr(accout), arr(base), arr(vout),
+                                      arr(copy), wc, wv, 0, 0), "bamhip_z4c_bc_rk4_stage")
+
+
+@pytest.mark.parametrize("shift", [0, 1, -1])
+def test_radiative_boundary_with_lists_crossed_between_fields(shift):
+    """an output that is the operand of the field `shift` places on: the values at the surface are those
+    of lists of their own, one product and one sum from the radiative right-hand side"""
+    size = (18, 15, 12)
+    par = B.z4c_params()
+    rng = np.random.default_rng(6)
+    ring = lambda lst: [lst[(v + shift) % 25] for v in range(25)]  # noqa: E731
+    lev, _, _ = _level(size)
+    lev.z4c_set_boundary(par, R, U)
+    k = lev.get_state(R)
+    on = ~_computed(size)
+    assert np.abs(k[:, on]).max() > 0
+    base, acc = rng.standard_normal((2,) + k.shape)
+    c, wc, wv = 0.4, 0.3, 0.7
+
+    def compare(lst, want, w):
+        bar = EPS * (np.abs(w * k) + np.abs(want))
+        assert (np.abs(lev.get_state(lst) - want)[:, on] <= bar[:, on]).all()
+
+    lev.put_state(P, base)
+    lev.z4c_set_boundary(par, ring(P), U, upre=P, c=c)
+    compare(ring(P), base + c * k, c)
+    lev.put_state(P, base)
+    lev.put_state(ACC, acc)
+    _bc_stage(lev, par, U, ACC, ring(ACC), P, ring(P), CP, wc, wv)
+    compare(ring(ACC), acc + wc * k, wc)
+    compare(ring(P), base + wv * k, wv)
+    compare(CP, base, 0.0)
+    lev.free()
+
+
+def test_radiative_boundary_into_one_variable_twice():
+    """a list that names a variable twice leaves the later field's value there"""
+    size = (9, 8, 10)
+    par = B.z4c_params()
+    lev, _, _ = _level(size)
+    lev.z4c_set_boundary(par, R, U)
+    k = lev.get_state(R)
+    lev.z4c_set_boundary(par, A[:24] + [A[3]], U)
+    got = lev.get_state(A)
+    k[3] = k[24]
+    k[24] = 0.0
+    on = ~_computed(size)
+    np.testing.assert_array_equal(got[:, on], k[:, on])
+    lev.free()
