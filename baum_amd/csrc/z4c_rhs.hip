@@ -696,8 +696,10 @@ struct TuneState {
 };
 static TuneState g_tune;
 
-static std::string region_signature(const RegionLists &R) {
-  std::string s;
+// the regions, and which stagings they admit: that depends on the whole level
+// (its size, the boxes' offsets) and not on the regions alone
+static std::string region_signature(const RegionLists &R, bool dma_ok, bool pairs_ok) {
+  std::string s = dma_ok ? pairs_ok ? "x4" : "x1" : "reg";
   char buf[96];
   for (const auto *v : R.kind) {
     s += '|';
@@ -729,7 +731,7 @@ static int choose_variant(int kind, const Z4cPtrs &P, const RegionLists &R, cons
       return set_error(BAMHIP_EINVAL, "z4c tile variant '%s' needs even box sizes and offsets", V[*idx].name);
     return BAMHIP_OK;
   }
-  const std::string sig = region_signature(R);
+  const std::string sig = region_signature(R, dma_ok, pairs_ok);
   auto it = g_tune.chosen[kind].find(sig);
   if (it != g_tune.chosen[kind].end()) {
     *idx = it->second.choice;

@@ -20,7 +20,7 @@ import pytest
 
 import baum_amd as B
 import oracle as O
-from spacetimes import grid, puncture_z4c
+from spacetimes import flat_z4c, grid, puncture_z4c
 
 pytestmark = pytest.mark.gpu
 
@@ -207,3 +207,30 @@ def test_radiative_boundary_into_one_variable_twice():
     on = ~_computed(size)
     np.testing.assert_array_equal(got[:, on], k[:, on])
     lev.free()
+
+
+@pytest.mark.parametrize("front", [((5, 5, 5), (1,) * 6), ((3, 3, 3), (2,) * 6)])
+def test_tuned_choice_is_not_taken_over_by_a_misaligned_level(front):
+    """a box of even rows admits the 16-byte staging, the same box behind an odd number of points does not:
+    the tuner times the second level anew, without it (x4=-1), also where the box in front has no regions"""
+    size, (fsize, fskip) = (24, 14, 16), front
+    lev, ob, u = _level(size)
+    cpu, _ = O.z4c_rhs(ob, O.z4c_params(), u)
+    fu = flat_z4c(fsize[::-1])
+    box = B.make_box(*size, ob.x0, ob.y0, ob.z0, ob.dx)
+    two = B.Level([B.make_box(*fsize, 5.0, 5.0, 5.0, ob.dx, skip=fskip), box], 50)
+    two.enable(range(50))
+    for v in R:
+        two.fill(v, 0.0)
+    two.put_state(U, np.concatenate([fu.reshape(25, -1), u.reshape(25, -1)], axis=1))
+    B.tune_clear()
+    lev.z4c_rhs(B.z4c_params(), R, U)
+    assert "x4=-1.0000ms" not in B.tune_report()
+    two.z4c_rhs(B.z4c_params(), R, U)
+    assert B.tune_report().count("x4=-1.0000ms") >= 1
+    got = two.box_view(two.get_state(R), 1)
+    floor = 64 / 12 * EPS * np.abs(u).max() / ob.dx ** 2
+    for v in range(25):
+        assert np.abs(got[v] - cpu[v]).max() <= max(1e-12 * np.abs(cpu[v]).max(), floor), B.VAR_NAMES[v]
+    lev.free()
+    two.free()
