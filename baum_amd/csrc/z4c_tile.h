@@ -917,10 +917,9 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
   });
 
   // ---- conformal factor
-  double df[3], K_, Theta;
+  double df[3];
+  const double Khat = pv[0], Theta = pv[1];
   {
-    const double Khat0 = pv[0];
-    Theta = pv[1];
     advance(std::integral_constant<int, 12>{}, nothing);
     double dchi[3], h6[6];
     const Fld F = field<SH, true, true>(T, G, w24, S, dchi, h6);
@@ -949,10 +948,10 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
         const int ab = sy(a, b);
         R[ab] += 4.0 * df[a] * df[b] - 2.0 * cddf[ab] - 2.0 * g[ab] * trcddf - 4.0 * g[ab] * dfdf;
       }
-    K_ = Khat0 + 2.0 * Theta;
     pin(R);
     pin(df);
-    emit(E[12 % 2], F.adv + eps * F.ko + (K.chipsipower / 6.0) * chig * (divbeta - alpha * K_));
+    emit(E[12 % 2],
+         F.adv + eps * F.ko + (K.chipsipower / 6.0) * chig * (divbeta - alpha * (Khat + 2.0 * Theta)));
   }
 
   // ---- lapse; after this stage sA holds the curvature terms of At_ij
@@ -961,7 +960,7 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
     advance(std::integral_constant<int, 13>{}, nothing);
     double cdda[6], h6[6];
     const Fld F = field<SH, true, true>(T, G, w24, S, da, h6);
-    emit(E[13 % 2], K.oplogwithshift * F.adv + eps * F.ko - fa * (K_ - 2.0 * Theta));
+    emit(E[13 % 2], K.oplogwithshift * F.adv + eps * F.ko - fa * Khat);
     const double dfda = contract(df, da);
 #pragma unroll
     for (int a = 0; a < 3; a++)
@@ -995,6 +994,7 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
     });
     double d[3];
     Fld F = field<SH, true, false>(T, G, w24, S, d, none6);
+    const double K_ = Khat + 2.0 * Theta;  // Khat alone is the lapse's source: K - 2 Theta would cancel
 #pragma unroll
     for (int a = 0; a < 3; a++)
       rG[a] -= (4.0 / 3.0) * alpha * (ig[sy(a, 0)] * d[0] + ig[sy(a, 1)] * d[1] + ig[sy(a, 2)] * d[2]);

@@ -234,3 +234,29 @@ def test_tuned_choice_is_not_taken_over_by_a_misaligned_level(front):
         assert np.abs(got[v] - cpu[v]).max() <= max(1e-12 * np.abs(cpu[v]).max(), floor), B.VAR_NAMES[v]
     lev.free()
     two.free()
+
+
+def _flat_level(size, fields=()):
+    """flat space with constant fields {index: value}, radiative faces"""
+    u = flat_z4c(size[::-1])
+    for v, x in fields:
+        u[v] = x
+    lev = B.Level([B.make_box(*size, 0.0, 0.0, 0.0, 0.1)], 75)
+    lev.enable(range(75))
+    for v in R + A:
+        lev.fill(v, 0.0)
+    lev.put_state(U, u.reshape(25, -1))
+    return lev, u
+
+
+def test_lapse_source_with_theta_far_above_khat():
+    """d_t alpha = -2 alpha Khat where |Theta| is a million times |Khat|: Khat is used as it is read, so a
+    product and its factor round, 2 eps; from K - 2 Theta it would carry eps Theta / Khat.  (The differences of
+    a lapse of few bits are 0.)"""
+    size, alpha, khat = (24, 14, 15), 0.75, 1.2345e-9
+    lev, _ = _flat_level(size, ((18, alpha), (13, khat), (17, 1e-3)))
+    lev.z4c_rhs(B.z4c_params(), R, U)
+    got = lev.get(R[18])[_computed(size)]
+    want = -2.0 * alpha * khat
+    assert np.abs(got - want).max() <= 2 * EPS * abs(want)
+    lev.free()
