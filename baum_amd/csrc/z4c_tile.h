@@ -729,10 +729,12 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
   };
   auto nothing = [] {};
   // the powers, while few registers are in use: psi^-4 = chi^(-4/chipsipower),
-  // chi itself in the usual chi = psi^-4, and the driver's alpha^p
+  // chi itself in the usual chi = psi^-4 (and not a number below 0, where the
+  // power has no value), and the driver's alpha^p
   double psim4 = ld(u[6]), betaF = 0.0;
   psim4 = (psim4 < K.chiDivFloor) ? K.chiDivFloor : psim4;
   if (K.chipsipower != -4.0) psim4 = exp(-4.0 * K.oocp * log(psim4));
+  else psim4 = (psim4 < 0.0) ? __builtin_nan("") : psim4;
   if (withB)
     betaF = K.shiftgammacoeff * (K.shiftalphapower == 0.0   ? 1.0
                                  : K.shiftalphapower == 1.0 ? alpha

@@ -260,3 +260,17 @@ def test_lapse_source_with_theta_far_above_khat():
     want = -2.0 * alpha * khat
     assert np.abs(got - want).max() <= 2 * EPS * abs(want)
     lev.free()
+
+
+@pytest.mark.parametrize("at", [(5, 6, 7), (1, 6, 7)])
+@pytest.mark.parametrize("params", [dict(), dict(advection_lopsided=0)])
+def test_negative_conformal_factor_is_reported(at, params):
+    """psi^-4 = chi^(-4 / chipsipower) of a chi below 0 is not a number, in the bulk and in the shell, in the
+    tile kernel and in the per-point kernel; a positive floor under chi makes it one"""
+    lev, u = _flat_level((16, 14, 15))
+    u[(6,) + at[::-1]] = -1e-3
+    lev.put(U[6], u[6])
+    with pytest.raises(B.BamhipError, match="non-finite"):
+        lev.z4c_rhs(B.z4c_params(**params), R, U)
+    lev.z4c_rhs(B.z4c_params(z4_chi_div_floor=1e-4, **params), R, U)
+    lev.free()
