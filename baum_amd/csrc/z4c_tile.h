@@ -739,9 +739,9 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
     betaF = K.shiftgammacoeff * (K.shiftalphapower == 0.0   ? 1.0
                                  : K.shiftalphapower == 1.0 ? alpha
                                                             : pow(alpha, K.shiftalphapower));
-  double fa = K.oploglapse * K.lapseharmonicf + K.harmoniclapse * alpha;
-  if (K.oploglapse2 != 0.0) fa += K.oploglapse2 * (8.0 / 3.0) / (3.0 - alpha);
-  fa *= alpha;
+  // the division also where its coefficient is 0: no value at alpha = 3
+  const double fa0 = K.oploglapse * K.lapseharmonicf + K.oploglapse2 * (8.0 / 3.0) / (3.0 - alpha);
+  double fa = (fa0 + K.harmoniclapse * alpha) * alpha;
   pin(psim4);
   pin(betaF);
   pin(fa);

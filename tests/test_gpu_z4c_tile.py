@@ -274,3 +274,15 @@ def test_negative_conformal_factor_is_reported(at, params):
         lev.z4c_rhs(B.z4c_params(**params), R, U)
     lev.z4c_rhs(B.z4c_params(z4_chi_div_floor=1e-4, **params), R, U)
     lev.free()
+
+
+@pytest.mark.parametrize("params", [dict(), dict(advection_lopsided=0)])
+def test_lapse_of_three_is_reported(params):
+    """the second slicing's 1 / (3 - alpha) has no value at alpha = 3, whatever its coefficient, in the tile
+    kernel as in the per-point kernel"""
+    lev, u = _flat_level((16, 14, 15))
+    u[18, 7, 6, 5] = 3.0
+    lev.put(U[18], u[18])
+    with pytest.raises(B.BamhipError, match="non-finite"):
+        lev.z4c_rhs(B.z4c_params(**params), R, U)
+    lev.free()
