@@ -133,32 +133,34 @@ template <int A, int O, class L>
 __device__ __forceinline__ double ax(TP<L> T) {
   return at<(A == 0 ? O : 0), (A == 1 ? O : 0), (A == 2 ? O : 0)>(T);
 }
-// The seven points of one axis through the point, as odd and even pairs:
-// d_k = f(k) - f(-k), s_k = f(k) + f(-k).
+// The seven points of one axis through the point, the inner ones also as odd
+// and even pairs: d_k = f(k) - f(-k), s_k = f(k) + f(-k).
 struct Line {
-  double d1, d2, d3, s1, s2, s3;
+  double d1, d2, s1, s2;
   double p[3], m[3];  // f(k), f(-k)
 };
 template <int A, class L>
 __device__ __forceinline__ Line t_line(TP<L> T) {
   const double m1 = ax<A, -1>(T), p1 = ax<A, 1>(T), m2 = ax<A, -2>(T), p2 = ax<A, 2>(T), m3 = ax<A, -3>(T),
                p3 = ax<A, 3>(T);
-  return {p1 - m1, p2 - m2, p3 - m3, p1 + m1, p2 + m2, p3 + m3, {p1, p2, p3}, {m1, m2, m3}};
+  return {p1 - m1, p2 - m2, p1 + m1, p2 + m2, {p1, p2, p3}, {m1, m2, m3}};
 }
 // Lop-sided advection, dissipation, first and second derivative along one
 // axis from the same pairs.  The upwind row of w = beta/h is
 //   w > 0: w/12 (-3 f(-1) - 10 f(0) + 18 f(1) - 6 f(2) + f(3)),
-//   w < 0: its mirror image,
-// and splits into parts odd and even in the offset,
-//   w/24 (21 d1 - 6 d2 + d3) + |w|/24 (15 s1 - 6 s2 + s3 - 20 f(0)),
-// so both signs of w share the pairs and no weight is kept per sign:
-// 16 FP64 operations for advection and dissipation together, where the two
-// one-sided rows took 17 and shared nothing with the derivatives.
+//   w < 0: its mirror image.
+// The points that both rows use, f(-1) and f(1), enter as parts odd and even in
+// the offset; of the outer ones the upwind side is selected, so the downwind
+// ones, which the row leaves out, do not enter at all (through odd and even
+// parts of their own they would cancel up to rounding only):
+//   w/12 (21/2 d1) + |w|/12 (f(3) - 6 f(2) + 15/2 s1 - 10 f(0)), f(k) upwind.
+// 13 FP64 operations and a select for advection and dissipation together,
+// where the two one-sided rows took 17 and shared nothing with the derivatives.
 template <int A>
-__device__ __forceinline__ double l_adv(const Line &l, double f0, double w24) {
-  const double odd = (l.d3 - 6.0 * l.d2) + 21.0 * l.d1;
-  const double even = (l.s3 - 6.0 * l.s2) + 15.0 * l.s1 - 20.0 * f0;
-  return w24 * odd + fabs(w24) * even;
+__device__ __forceinline__ double l_adv(const Line &l, double f0, double w12) {
+  const double p = l.p[2] - 6.0 * l.p[1], m = l.m[2] - 6.0 * l.m[1];
+  const double up = w12 > 0.0 ? p : m;
+  return w12 * (10.5 * l.d1) + fabs(w12) * ((up + 7.5 * l.s1) - 10.0 * f0);
 }
 template <int A>
 __device__ __forceinline__ double l_ko(const Line &l, double f0, const Z4cGeo &G) {
@@ -180,10 +182,10 @@ __device__ __forceinline__ double l_d2(const Line &l, double f0, const Z4cGeo &G
 // it as coefficients set once per point, so the shell reads the same neighbours
 // at fixed LDS offsets as the bulk and has no branch: a neighbour outside the
 // box is read with coefficient 0 from a staging slot that holds box data.  (The
-// advection takes one coefficient per neighbour: its odd and even parts, as the
-// bulk sums them, would cancel a neighbour only up to rounding.  A branch on the point's order inside a
-// stage also let the register allocator place copies of live values where only
-// part of the wave was enabled.)
+// advection takes one coefficient per neighbour: its rows are more than the two
+// of the bulk.  A branch on the point's order inside a stage also let the
+// register allocator place copies of live values where only part of the wave was
+// enabled.)
 //   order 4 (e = 1) / order 2 (e = 0):
 //     first derivative  ((6 + 2 e) d1 - e d2) / (12 h)
 //     second            ((12 + 4 e) s1 - e s2 - (24 + 6 e) f) / (12 h^2)
@@ -198,7 +200,7 @@ struct Sten {
 };
 
 // pos: distances (low, high) of the point to the box's edges per axis
-__device__ __forceinline__ void set_sten(Sten &S, const int dl[3], const int dh[3], const double w24[3]) {
+__device__ __forceinline__ void set_sten(Sten &S, const int dl[3], const int dh[3], const double w12[3]) {
   int dmin = 1 << 30;
 #pragma unroll
   for (int a = 0; a < 3; a++) dmin = min(dmin, min(dl[a], dh[a]));
@@ -213,20 +215,20 @@ __device__ __forceinline__ void set_sten(Sten &S, const int dl[3], const int dh[
   S.a0 = 0.0;
 #pragma unroll
   for (int a = 0; a < 3; a++) {
-    const double aw = fabs(w24[a]);
-    const bool pos = w24[a] > 0.0, up = (pos ? dh[a] : dl[a]) >= (o4 ? 3 : 2);
-    const double f1 = aw * (o4 ? (up ? 36.0 : 16.0) : (up ? 48.0 : 12.0));
-    const double f2 = aw * (o4 ? (up ? -12.0 : -2.0) : (up ? -12.0 : 0.0));
-    const double f3 = aw * (o4 && up ? 2.0 : 0.0);
-    const double b1 = aw * (o4 ? (up ? -6.0 : -16.0) : (up ? 0.0 : -12.0));
-    const double b2 = aw * (o4 && !up ? 2.0 : 0.0);
+    const double aw = fabs(w12[a]);
+    const bool pos = w12[a] > 0.0, up = (pos ? dh[a] : dl[a]) >= (o4 ? 3 : 2);
+    const double f1 = aw * (o4 ? (up ? 18.0 : 8.0) : (up ? 24.0 : 6.0));
+    const double f2 = aw * (o4 ? (up ? -6.0 : -1.0) : (up ? -6.0 : 0.0));
+    const double f3 = aw * (o4 && up ? 1.0 : 0.0);
+    const double b1 = aw * (o4 ? (up ? -3.0 : -8.0) : (up ? 0.0 : -6.0));
+    const double b2 = aw * (o4 && !up ? 1.0 : 0.0);
     S.ap[a][0] = pos ? f1 : b1;
     S.ap[a][1] = pos ? f2 : b2;
     S.ap[a][2] = pos ? f3 : 0.0;
     S.am[a][0] = pos ? b1 : f1;
     S.am[a][1] = pos ? b2 : f2;
     S.am[a][2] = pos ? 0.0 : f3;
-    S.a0 += aw * (up ? (o4 ? -20.0 : -36.0) : 0.0);
+    S.a0 += aw * (up ? (o4 ? -10.0 : -18.0) : 0.0);
   }
 }
 
@@ -248,11 +250,11 @@ __device__ __forceinline__ double t_mixed(TP<L> T, const Z4cGeo &G, const Sten &
 }
 // advection, dissipation, first and second derivative along one axis
 template <bool SH, int A>
-__device__ __forceinline__ double s_adv(const Line &l, double f0, double w24, const Sten &S) {
+__device__ __forceinline__ double s_adv(const Line &l, double f0, double w12, const Sten &S) {
   if constexpr (SH)
     return S.ap[A][0] * l.p[0] + S.ap[A][1] * l.p[1] + S.ap[A][2] * l.p[2] + S.am[A][0] * l.m[0] +
            S.am[A][1] * l.m[1] + S.am[A][2] * l.m[2];
-  return l_adv<A>(l, f0, w24);
+  return l_adv<A>(l, f0, w12);
 }
 template <bool SH, int A>
 __device__ __forceinline__ double s_d1(const Line &l, const Z4cGeo &G, const Sten &S) {
@@ -271,25 +273,25 @@ struct Fld {
   double f0, adv, ko;
 };
 template <bool SH, bool GRAD, bool HESS, class L>
-__device__ __forceinline__ Fld field(TP<L> T, const Z4cGeo &G, const double w24[3], const Sten &S, double d[3],
+__device__ __forceinline__ Fld field(TP<L> T, const Z4cGeo &G, const double w12[3], const Sten &S, double d[3],
                                      double h6[6]) {
   Fld F;
   F.f0 = ax<0, 0>(T);
   const Line x = t_line<0>(T);
-  F.adv = s_adv<SH, 0>(x, F.f0, w24[0], S);
+  F.adv = s_adv<SH, 0>(x, F.f0, w12[0], S);
   if constexpr (SH) F.adv = F.adv + S.a0 * F.f0;
   F.ko = l_ko<0>(x, F.f0, G);
   if constexpr (GRAD) d[0] = s_d1<SH, 0>(x, G, S);
   if constexpr (HESS) h6[0] = s_d2<SH, 0>(x, F.f0, G, S);
   BH_PHASE();
   const Line y = t_line<1>(T);
-  F.adv += s_adv<SH, 1>(y, F.f0, w24[1], S);
+  F.adv += s_adv<SH, 1>(y, F.f0, w12[1], S);
   F.ko += l_ko<1>(y, F.f0, G);
   if constexpr (GRAD) d[1] = s_d1<SH, 1>(y, G, S);
   if constexpr (HESS) h6[3] = s_d2<SH, 1>(y, F.f0, G, S);
   BH_PHASE();
   const Line z = t_line<2>(T);
-  F.adv += s_adv<SH, 2>(z, F.f0, w24[2], S);
+  F.adv += s_adv<SH, 2>(z, F.f0, w12[2], S);
   F.ko = -(F.ko + l_ko<2>(z, F.f0, G));
   if constexpr (SH) F.ko *= S.kof;
   if constexpr (GRAD) d[2] = s_d1<SH, 2>(z, G, S);
@@ -651,16 +653,16 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
   // before its use.  (A thread without a point of its own loads the block's
   // first point; its results are not stored.)
   const bool withB = K.withB != 0.0;
-  double g[6], w24[3];
+  double g[6], w12[3];
   double pv[2];  // point values loaded a stage before their use
 #pragma unroll
   for (int c = 0; c < 6; c++) g[c] = ld(u[c]);
 #pragma unroll
-  for (int a = 0; a < 3; a++) w24[a] = ld(u[19 + a]) * G.ih[a] * (1.0 / 24.0);
+  for (int a = 0; a < 3; a++) w12[a] = ld(u[19 + a]) * G.ih[a] * (1.0 / 12.0);
   const double alpha = ld(u[18]);
   pv[0] = ld(withB ? u[22] : u[14]);
   Sten S{};
-  if constexpr (SH) set_sten(S, dl, dh, w24);
+  if constexpr (SH) set_sten(S, dl, dh, w12);
   // Memory traffic of a stage, in the order it is issued right after the
   // stage's barrier: the loads of this stage's store operands (an RK4 stage's
   // accumulator and start state, or upre) and of the point values the next
@@ -781,7 +783,7 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
         else pv[0] = ld(u[7]);
       });
       double d[3], h6[6];
-      const Fld F = field<SH, true, true>(T, G, w24, S, d, h6);
+      const Fld F = field<SH, true, true>(T, G, w12, S, d, h6);
 #pragma unroll
       for (int a = 0; a < 3; a++) {
         db[a][c] = d[a];
@@ -817,7 +819,7 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
         if constexpr (ab < 5) pv[0] = ld(u[8 + ab]);
       });
       double d[3], h6[6];
-      const Fld F = field<SH, true, true>(T, G, w24, S, d, h6);
+      const Fld F = field<SH, true, true>(T, G, w12, S, d, h6);
 #pragma unroll
       for (int e = 0; e < 3; e++) {
         dg[e][ab] = d[e];
@@ -906,7 +908,7 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
       }
     });
     double dG[3];
-    const Fld F = field<SH, true, false>(T, G, w24, S, dG, none6);
+    const Fld F = field<SH, true, false>(T, G, w12, S, dG, none6);
 #pragma unroll
     for (int a = 0; a < 3; a++)
 #pragma unroll
@@ -924,7 +926,7 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
   {
     advance(std::integral_constant<int, 12>{}, nothing);
     double dchi[3], h6[6];
-    const Fld F = field<SH, true, true>(T, G, w24, S, dchi, h6);
+    const Fld F = field<SH, true, true>(T, G, w12, S, dchi, h6);
     const double chi = F.f0;
     const double chig = (chi < K.chiDivFloor) ? K.chiDivFloor : chi;
     const double oochig = 1.0 / chig;
@@ -961,7 +963,7 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
   {
     advance(std::integral_constant<int, 13>{}, nothing);
     double cdda[6], h6[6];
-    const Fld F = field<SH, true, true>(T, G, w24, S, da, h6);
+    const Fld F = field<SH, true, true>(T, G, w12, S, da, h6);
     emit(E[13 % 2], K.oplogwithshift * F.adv + eps * F.ko - fa * Khat);
     const double dfda = contract(df, da);
 #pragma unroll
@@ -995,7 +997,7 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
       for (int c = 0; c < 6; c++) A[c] = ld(u[7 + c]);
     });
     double d[3];
-    Fld F = field<SH, true, false>(T, G, w24, S, d, none6);
+    Fld F = field<SH, true, false>(T, G, w12, S, d, none6);
     const double K_ = Khat + 2.0 * Theta;  // Khat alone is the lapse's source: K - 2 Theta would cancel
 #pragma unroll
     for (int a = 0; a < 3; a++)
@@ -1041,7 +1043,7 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
   {
     double d[3];
     advance(std::integral_constant<int, 15>{}, nothing);
-    const Fld F = field<SH, true, false>(T, G, w24, S, d, none6);
+    const Fld F = field<SH, true, false>(T, G, w12, S, d, none6);
 #pragma unroll
     for (int a = 0; a < 3; a++)
       rG[a] -= (2.0 / 3.0) * alpha * (ig[sy(a, 0)] * d[0] + ig[sy(a, 1)] * d[1] + ig[sy(a, 2)] * d[2]);
@@ -1054,7 +1056,7 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
   static_for<6>([&](auto I_) {
     constexpr int ab = decltype(I_)::value;
     advance(std::integral_constant<int, 16 + ab>{}, nothing);
-    const Fld F = field<SH, false, false>(T, G, w24, S, none3, none6);
+    const Fld F = field<SH, false, false>(T, G, w12, S, none3, none6);
     emit(E[(16 + ab) % 2], F.adv + eps * F.ko + sA[ab]);
     if constexpr (ab < 3) emit(Q[(16 + ab) % 2], rG[ab] + park[ab * NTHR + tid]);
   });
@@ -1063,7 +1065,7 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
   static_for<3>([&](auto I_) {
     constexpr int c = decltype(I_)::value;
     advance(std::integral_constant<int, 22 + c>{}, nothing);
-    const Fld F = field<SH, false, false>(T, G, w24, S, none3, none6);
+    const Fld F = field<SH, false, false>(T, G, w12, S, none3, none6);
     const double drive = K.withBadv * F.adv + ((K.gamma0factor + K.gamma2factor * betaF) *
                                                    (rG[c] - park[(3 + c) * NTHR + tid]) -
                                                K.shiftdriver * F.f0);

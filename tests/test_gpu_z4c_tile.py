@@ -286,3 +286,30 @@ def test_lapse_of_three_is_reported(params):
     with pytest.raises(B.BamhipError, match="non-finite"):
         lev.z4c_rhs(B.z4c_params(**params), R, U)
     lev.free()
+
+
+@pytest.mark.parametrize("signs", [(1, 1, 1), (-1, -1, -1), (1, -1, 1)])
+def test_upwind_row_leaves_out_the_downwind_points(signs):
+    """the lop-sided row of a shift component reaches three points upwind and one downwind: a spike anywhere
+    else changes nothing, not by rounding either.  B is advected and read at the point, nothing more."""
+    size, spike = (24, 14, 15), (11, 7, 7)
+    par = dict(z4_shift="withB gamma0 withGadv withBadv withShiftadv", order_dissipation=0)
+    rng = np.random.default_rng(8)
+    lev, u = _flat_level(size, tuple((19 + a, 0.3 * s) for a, s in enumerate(signs)))
+    u[22:25] = rng.standard_normal((3,) + size[::-1])
+    ob = O.make_box(*size, 0.0, 0.0, 0.0, 0.1, skip=(1,) * 6)
+    out, ref = [], []
+    for value in (0.0, 1e10):
+        u[(slice(22, 25),) + spike[::-1]] = value
+        lev.put_state(U, u.reshape(25, -1))
+        lev.z4c_rhs(B.z4c_params(**par), R, U)
+        out.append(lev.get_state(R)[22:].reshape((3,) + size[::-1]))
+        ref.append(O.z4c_rhs(ob, O.z4c_params(**par), u)[0][22:])
+    same = ref[0] == ref[1]
+    for a in range(3):  # the points that see the spike two and three points downwind
+        for d in (2, 3):
+            q = list(spike)
+            q[a] += d * signs[a]
+            assert same[(slice(None),) + tuple(q[::-1])].all()
+    np.testing.assert_array_equal(out[1][same], out[0][same])
+    lev.free()
