@@ -179,24 +179,24 @@ __device__ __forceinline__ double l_d2(const Line &l, double f0, const Z4cGeo &G
 // centred differences and order-2 advection rows, dissipation needs two or
 // more points to every edge, and the advection row is the upwind one where it
 // fits between the point and the edge and the centred one elsewhere.  All of
-// it as coefficients set once per point, so the shell reads the same neighbours
-// at fixed LDS offsets as the bulk and has no branch: a neighbour outside the
-// box is read with coefficient 0 from a staging slot that holds box data.  (The
-// advection takes one coefficient per neighbour: its rows are more than the two
-// of the bulk.  A branch on the point's order inside a stage also let the
-// register allocator place copies of live values where only part of the wave was
-// enabled.)
+// it as coefficients set once per point and selects, so the shell reads the same
+// neighbours at fixed LDS offsets as the bulk and has no branch (one inside a
+// stage let the register allocator place copies of live values where only part
+// of the wave was enabled).  What an order-2 derivative leaves out is selected
+// away, not multiplied by 0: it may hold anything.  The advection takes one
+// coefficient per neighbour, 0 for one that its row leaves out; a neighbour
+// outside the box is read from a staging slot that holds 0 or box data.
 //   order 4 (e = 1) / order 2 (e = 0):
 //     first derivative  ((6 + 2 e) d1 - e d2) / (12 h)
 //     second            ((12 + 4 e) s1 - e s2 - (24 + 6 e) f) / (12 h^2)
-//     mixed             ((36 + 28 e) q11 - 8 e (q12 + q21) + e q22) / (144 h h')
+//     mixed             ((36 + 28 e) q11 + e (q22 - 8 (q12 + q21))) / (144 h h')
 //     advection, w = beta / h, f(k) counted in the direction of w:
 //       upwind   |w|/12 (-3 f(-1) - 10 f(0) + 18 f(1) - 6 f(2) + f(3)),  |w|/2 (-3 f(0) + 4 f(1) - f(2))
 //       centred  |w|/12 (8 (f(1) - f(-1)) - (f(2) - f(-2))),             |w|/2 (f(1) - f(-1))
 struct Sten {
-  double e, c1, p1, p0, k1, k2;   // the coefficients above: e, 6 + 2e, 12 + 4e, 24 + 6e, 36 + 28e, 8e
+  bool o4;                        // order 4, and dissipation on
+  double c1, p1, p0, k1;          // the coefficients above: 6 + 2e, 12 + 4e, 24 + 6e, 36 + 28e
   double ap[3][3], am[3][3], a0;  // advection: coefficients of f(1..3) and f(-1..-3) per axis, and of f
-  double kof;                     // 1 where dissipation is on, else 0
 };
 
 // pos: distances (low, high) of the point to the box's edges per axis
@@ -204,14 +204,11 @@ __device__ __forceinline__ void set_sten(Sten &S, const int dl[3], const int dh[
   int dmin = 1 << 30;
 #pragma unroll
   for (int a = 0; a < 3; a++) dmin = min(dmin, min(dl[a], dh[a]));
-  const bool o4 = dmin >= 2;
-  S.e = o4 ? 1.0 : 0.0;
+  const bool o4 = S.o4 = dmin >= 2;
   S.c1 = o4 ? 8.0 : 6.0;
   S.p1 = o4 ? 16.0 : 12.0;
   S.p0 = o4 ? 30.0 : 24.0;
   S.k1 = o4 ? 64.0 : 36.0;
-  S.k2 = o4 ? 8.0 : 0.0;
-  S.kof = o4 ? 1.0 : 0.0;
   S.a0 = 0.0;
 #pragma unroll
   for (int a = 0; a < 3; a++) {
@@ -245,8 +242,9 @@ template <bool SH, int A, int B, class L>
 __device__ __forceinline__ double t_mixed(TP<L> T, const Z4cGeo &G, const Sten &S) {
   const double q11 = t_corner<A, B, 1, 1>(T), q12 = t_corner<A, B, 1, 2>(T), q21 = t_corner<A, B, 2, 1>(T),
                q22 = t_corner<A, B, 2, 2>(T);
-  if constexpr (SH) return ((S.e * q22 - S.k2 * (q12 + q21)) + S.k1 * q11) * G.i144hh[A + B - 1];
-  return ((q22 - 8.0 * (q12 + q21)) + 64.0 * q11) * G.i144hh[A + B - 1];
+  const double outer = q22 - 8.0 * (q12 + q21);
+  if constexpr (SH) return ((S.o4 ? outer : 0.0) + S.k1 * q11) * G.i144hh[A + B - 1];
+  return (outer + 64.0 * q11) * G.i144hh[A + B - 1];
 }
 // advection, dissipation, first and second derivative along one axis
 template <bool SH, int A>
@@ -258,12 +256,12 @@ __device__ __forceinline__ double s_adv(const Line &l, double f0, double w12, co
 }
 template <bool SH, int A>
 __device__ __forceinline__ double s_d1(const Line &l, const Z4cGeo &G, const Sten &S) {
-  if constexpr (SH) return (S.c1 * l.d1 - S.e * l.d2) * G.i12h[A];
+  if constexpr (SH) return (S.c1 * l.d1 - (S.o4 ? l.d2 : 0.0)) * G.i12h[A];
   return l_d1<A>(l, G);
 }
 template <bool SH, int A>
 __device__ __forceinline__ double s_d2(const Line &l, double f0, const Z4cGeo &G, const Sten &S) {
-  if constexpr (SH) return ((S.p1 * l.s1 - S.e * l.s2) - S.p0 * f0) * G.i12hh[A];
+  if constexpr (SH) return ((S.p1 * l.s1 - (S.o4 ? l.s2 : 0.0)) - S.p0 * f0) * G.i12hh[A];
   return l_d2<A>(l, f0, G);
 }
 
@@ -293,7 +291,7 @@ __device__ __forceinline__ Fld field(TP<L> T, const Z4cGeo &G, const double w12[
   const Line z = t_line<2>(T);
   F.adv += s_adv<SH, 2>(z, F.f0, w12[2], S);
   F.ko = -(F.ko + l_ko<2>(z, F.f0, G));
-  if constexpr (SH) F.ko *= S.kof;
+  if constexpr (SH) F.ko = S.o4 ? F.ko : 0.0;
   if constexpr (GRAD) d[2] = s_d1<SH, 2>(z, G, S);
   if constexpr (HESS) {
     h6[5] = s_d2<SH, 2>(z, F.f0, G, S);
@@ -361,7 +359,7 @@ struct Stager {
       ok |= in ? (1u << k) : 0u;
     }
   }
-  // slots outside the box are staged as 0; no stencil of a computed point reads them
+  // slots outside the box are staged as 0; a stencil has coefficient 0 there or selects them away
   __device__ __forceinline__ void load(const double *__restrict__ f) {
 #pragma unroll
     for (int k = 0; k < NLOAD; k++) pf[k] = (ok >> k & 1u) ? f[cbase + goff[k]] : 0.0;

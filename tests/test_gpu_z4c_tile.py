@@ -313,3 +313,22 @@ def test_upwind_row_leaves_out_the_downwind_points(signs):
             assert same[(slice(None),) + tuple(q[::-1])].all()
     np.testing.assert_array_equal(out[1][same], out[0][same])
     lev.free()
+
+
+@pytest.mark.parametrize("field", [0, 6, 18, 19])
+@pytest.mark.parametrize("off", [(1, 2, 0), (2, 1, 0), (-1, -2, 0), (0, 1, 2), (0, -2, 2), (1, 0, -2)])
+def test_order_two_points_do_not_read_the_outer_corners(field, off):
+    """one point from a face the mixed derivatives are of order 2 and reach one point: what lies further out
+    off the axes does not matter, not even when it is no number"""
+    size, at = (16, 14, 15), (1, 7, 6)
+    lev, _, u = _level(size)
+    lev.set_check(0)
+    q = at[0] + size[0] * (at[1] + size[1] * at[2])
+    lev.z4c_rhs(B.z4c_params(), R, U)
+    want = lev.get_state(R)[:, q]
+    u[(field,) + tuple(np.add(at, off))[::-1]] = np.nan
+    lev.put(U[field], u[field])
+    lev.z4c_rhs(B.z4c_params(), R, U)
+    np.testing.assert_array_equal(lev.get_state(R)[:, q], want)
+    assert np.isfinite(want).all()
+    lev.free()
