@@ -663,8 +663,9 @@ static int plan_box(const DevBox &B, const Z4cPtrs &P, const Z4cK &K, int *flag,
 
 // ---- autotuner of the tile kernels
 // A variant is one staging of the tile kernel: through registers, or by
-// LDS-DMA in dwords or in 16-byte units.  Every variant evaluates the same per-point arithmetic in the same
-// order, so all give bitwise the same right-hand side.  The first time a set
+// LDS-DMA in dwords or in 16-byte units.  Every variant evaluates the same
+// per-point arithmetic in the same order, so all give bitwise the same
+// right-hand side.  The first time a set
 // of regions (a level's boxes) is seen outside graph capture, each variant is
 // timed on it (one warm-up launch, then two timed with HIP events) and the
 // fastest is kept for that set.
@@ -681,8 +682,11 @@ static const Variant kVariants[2][kMaxVariants] = {{{"bulk 16x4x4 dma3", true, f
                                                    {{"shell slabs dma3", true, false, tile_dma},
                                                     {"shell slabs reg", false, false, tile_reg},
                                                     {"shell slabs dma3 x4", true, true, tile_dma_x4}}};
-static const int kNumVariants[2] = {3, 3};
 // variant 0 of each kind is the default; variant 1 needs no LDS-DMA
+// The variant behind each public index: tile shapes, numbers of buffers and
+// thread orders that had indices of their own now share their staging's kernel.
+static const int kNumIndex[2] = {9, 6};
+static const int kVariantOf[2][9] = {{0, 1, 0, 0, 0, 2, 2, 2, 0}, {0, 1, 0, 0, 2, 2}};
 
 struct TuneEntry {
   int choice;
@@ -721,7 +725,6 @@ static std::string region_signature(const RegionLists &R, bool dma_ok, bool pair
 static int choose_variant(int kind, const Z4cPtrs &P, const RegionLists &R, const Z4cK &K, int *flag,
                           bool repeatable, bool dma_ok, bool pairs_ok, int *idx, bool *done) {
   const Variant *V = kVariants[kind];
-  const int nv = kNumVariants[kind];
   *done = false;
   *idx = g_tune.forced[kind];
   if (*idx >= 0) {
@@ -749,7 +752,7 @@ static int choose_variant(int kind, const Z4cPtrs &P, const RegionLists &R, cons
   BH_HIP(hipEventCreate(&b));
   double best = 1e300;
   int e = BAMHIP_OK;
-  for (int v = 0; v < nv && e == BAMHIP_OK; v++) {
+  for (int v = 0; v < kMaxVariants && e == BAMHIP_OK; v++) {
     te.ms[v] = -1.0;
     if ((V[v].dma && !dma_ok) || (V[v].pairs && !pairs_ok)) continue;
     if ((e = V[v].fn(P, R, K, flag, stream()))) break;
@@ -1015,21 +1018,21 @@ extern "C" int bamhip_z4c_tune_clear(void) {
 
 extern "C" int bamhip_z4c_variant_count(int kind) {
   if (kind != 0 && kind != 1) return bamhip::set_error(BAMHIP_EINVAL, "bamhip_z4c_variant_count: kind %d", kind);
-  return bamhip::kNumVariants[kind];
+  return bamhip::kNumIndex[kind];
 }
 
 extern "C" const char *bamhip_z4c_variant_name(int kind, int idx) {
   if (kind != 0 && kind != 1) return nullptr;
-  if (idx < 0 || idx >= bamhip::kNumVariants[kind]) return nullptr;
-  return bamhip::kVariants[kind][idx].name;
+  if (idx < 0 || idx >= bamhip::kNumIndex[kind]) return nullptr;
+  return bamhip::kVariants[kind][bamhip::kVariantOf[kind][idx]].name;
 }
 
 extern "C" int bamhip_z4c_force_variant(int kind, int idx) {
   if (kind != 0 && kind != 1) return bamhip::set_error(BAMHIP_EINVAL, "bamhip_z4c_force_variant: kind %d", kind);
-  if (idx < -1 || idx >= bamhip::kNumVariants[kind])
+  if (idx < -1 || idx >= bamhip::kNumIndex[kind])
     return bamhip::set_error(BAMHIP_EINVAL, "bamhip_z4c_force_variant: variant %d of %d", idx,
-                             bamhip::kNumVariants[kind]);
-  bamhip::g_tune.forced[kind] = idx;
+                             bamhip::kNumIndex[kind]);
+  bamhip::g_tune.forced[kind] = idx < 0 ? -1 : bamhip::kVariantOf[kind][idx];
   return BAMHIP_OK;
 }
 
@@ -1042,7 +1045,7 @@ extern "C" int bamhip_z4c_tune_report(char *buf, int len) {
       snprintf(line, sizeof line, "%s <- %zu regions:", bamhip::kVariants[kind][te.choice].name,
                (size_t)std::count(kv.first.begin(), kv.first.end(), ';'));
       s += line;
-      for (int v = 0; v < bamhip::kNumVariants[kind]; v++) {
+      for (int v = 0; v < bamhip::kMaxVariants; v++) {
         snprintf(line, sizeof line, " %s=%.4fms", bamhip::kVariants[kind][v].name, te.ms[v]);
         s += line;
       }

@@ -160,13 +160,14 @@ int bamhip_z4c_rhs(bamhip_level *lev, const bamhip_z4c_params *par,
 /* Autotuner of the RHS tile kernels (no counterpart in the reference, whose
  * RHS is one OpenMP loop nest, z4_rhs_movpunc_N.c:23).  kind 0: the bulk
  * kernel (points >= 3 from every box edge); kind 1: the box-edge shell.
- * A variant fixes the tile shape (its z depth included) and the LDS staging;
- * all variants give bitwise the same RHS.  In mode 1 (default) the first
- * bamhip_z4c_rhs call on a new set of boxes, outside graph capture and with
- * unew not aliasing upre, times every variant and keeps the fastest for that
- * set; mode 0 uses variant 0.  bamhip_z4c_force_variant(kind, i) pins variant
- * i (-1: back to the tuner).  tune_report writes one line per tuned set with
- * the time of each variant and returns the length needed (with the NUL). */
+ * A variant fixes the LDS staging (several of the nine bulk and six shell
+ * indices name the same one); all variants give bitwise the same RHS.  In
+ * mode 1 (default) the first bamhip_z4c_rhs call on a new set of boxes,
+ * outside graph capture and with unew not aliasing upre, times every variant
+ * and keeps the fastest for that set; mode 0 uses variant 0.
+ * bamhip_z4c_force_variant(kind, i) pins variant i (-1: back to the tuner).
+ * tune_report writes one line per tuned set with the time of each variant and
+ * returns the length needed (with the NUL). */
 int bamhip_z4c_tune_mode(int mode);
 /* on != 0 (default): the bulk and box-edge shell tiles of a level run in one
  * launch where both are staged the same way, else one after the other; returns

@@ -332,3 +332,26 @@ def test_order_two_points_do_not_read_the_outer_corners(field, off):
     np.testing.assert_array_equal(lev.get_state(R)[:, q], want)
     assert np.isfinite(want).all()
     lev.free()
+
+
+def test_every_index_of_a_variant_can_be_pinned():
+    """nine bulk and six shell indices, several of which share a kernel: each gives bitwise the same"""
+    lev, _, _ = _level((24, 14, 16))
+    names = [B.variants(k) for k in (B.BULK, B.SHELL)]
+    assert [len(n) for n in names] == [9, 6] and [len(set(n)) for n in names] == [3, 3]
+    first = None
+    try:
+        for kind in (B.BULK, B.SHELL):
+            for v in range(len(names[kind])):
+                B.force_variant(kind, v)
+                lev.z4c_rhs(B.z4c_params(), R, U)
+                got = lev.get_state(R)
+                first = got if first is None else first
+                np.testing.assert_array_equal(got, first)
+            B.force_variant(kind, -1)
+            with pytest.raises(B.BamhipError):
+                B.force_variant(kind, len(names[kind]))
+    finally:
+        B.force_variant(B.BULK, -1)
+        B.force_variant(B.SHELL, -1)
+    lev.free()
