@@ -665,10 +665,14 @@ static int plan_box(const DevBox &B, const Z4cPtrs &P, const Z4cK &K, int *flag,
 // A variant is one staging of the tile kernel: through registers, or by
 // LDS-DMA in dwords or in 16-byte units.  Every variant evaluates the same
 // per-point arithmetic in the same order, so all give bitwise the same
-// right-hand side.  The first time a set
-// of regions (a level's boxes) is seen outside graph capture, each variant is
-// timed on it (one warm-up launch, then two timed with HIP events) and the
-// fastest is kept for that set.
+// right-hand side.  The first time a level's boxes are seen outside graph
+// capture, each launch that may run is timed on them with every variant (one
+// warm-up launch, then two timed with HIP events): the bulk tiles, the slabs of
+// the box-edge shell, and both in one launch.  A level with bulk and shell takes
+// one launch unless two, each with its own fastest variant, took less: the
+// kernel of all four bodies is larger and spills more than that of the bulk
+// alone, but leaves no tail between the two.  (Timed on the two launches only,
+// the choice said nothing of the one that ran.)
 struct Variant {
   const char *name;
   bool dma;    // LDS-DMA staging: byte offsets within a field must fit 32 bits
@@ -676,27 +680,32 @@ struct Variant {
   LaunchFn fn;
 };
 constexpr int kMaxVariants = 3;
-static const Variant kVariants[2][kMaxVariants] = {{{"bulk 16x4x4 dma3", true, false, tile_dma},
-                                                    {"bulk 16x4x4 reg", false, false, tile_reg},
-                                                    {"bulk 16x4x4 dma3 x4", true, true, tile_dma_x4}},
-                                                   {{"shell slabs dma3", true, false, tile_dma},
-                                                    {"shell slabs reg", false, false, tile_reg},
-                                                    {"shell slabs dma3 x4", true, true, tile_dma_x4}}};
-// variant 0 of each kind is the default; variant 1 needs no LDS-DMA
+enum { kBulk, kShell, kBoth, kLaunches };
+static const Variant kVariants[kLaunches][kMaxVariants] = {{{"bulk 16x4x4 dma3", true, false, tile_dma},
+                                                            {"bulk 16x4x4 reg", false, false, tile_reg},
+                                                            {"bulk 16x4x4 dma3 x4", true, true, tile_dma_x4}},
+                                                           {{"shell slabs dma3", true, false, tile_dma},
+                                                            {"shell slabs reg", false, false, tile_reg},
+                                                            {"shell slabs dma3 x4", true, true, tile_dma_x4}},
+                                                           {{"one launch dma3", true, false, tile_dma},
+                                                            {"one launch reg", false, false, tile_reg},
+                                                            {"one launch dma3 x4", true, true, tile_dma_x4}}};
+// variant 0 is the default; variant 1 needs no LDS-DMA
 // The variant behind each public index: tile shapes, numbers of buffers and
 // thread orders that had indices of their own now share their staging's kernel.
 static const int kNumIndex[2] = {9, 6};
 static const int kVariantOf[2][9] = {{0, 1, 0, 0, 0, 2, 2, 2, 0}, {0, 1, 0, 0, 2, 2}};
 
 struct TuneEntry {
-  int choice;
-  double ms[kMaxVariants];
+  int choice[kLaunches];               // fastest variant, -1: no such tiles
+  double ms[kLaunches][kMaxVariants];  // -1: not admissible
+  bool one;                            // bulk and shell in one launch
 };
 struct TuneState {
   int overlap = 1;  // shell and bulk tiles in one launch
   int mode = 1;  // 0: defaults only; 1: tune each new region set
   int forced[2] = {-1, -1};
-  std::map<std::string, TuneEntry> chosen[2];
+  std::map<std::string, TuneEntry> chosen;
 };
 static TuneState g_tune;
 
@@ -717,43 +726,16 @@ static std::string region_signature(const RegionLists &R, bool dma_ok, bool pair
   return s;
 }
 
-// Variant of kind for the region lists R: the pinned one, the one kept for
-// this region set, or (mode 1, outside capture, repeatable launches) the
-// fastest after timing all of them on the library stream.  In the last case
-// the chosen variant has also been run once more, so the outputs are in place
-// and *done is set.
-static int choose_variant(int kind, const Z4cPtrs &P, const RegionLists &R, const Z4cK &K, int *flag,
-                          bool repeatable, bool dma_ok, bool pairs_ok, int *idx, bool *done) {
-  const Variant *V = kVariants[kind];
-  *done = false;
-  *idx = g_tune.forced[kind];
-  if (*idx >= 0) {
-    if (V[*idx].dma && !dma_ok)
-      return set_error(BAMHIP_EINVAL, "z4c tile variant '%s' needs a level below 2^29 points", V[*idx].name);
-    if (V[*idx].pairs && !pairs_ok)
-      return set_error(BAMHIP_EINVAL, "z4c tile variant '%s' needs even box sizes and offsets", V[*idx].name);
-    return BAMHIP_OK;
-  }
-  const std::string sig = region_signature(R, dma_ok, pairs_ok);
-  auto it = g_tune.chosen[kind].find(sig);
-  if (it != g_tune.chosen[kind].end()) {
-    *idx = it->second.choice;
-    return BAMHIP_OK;
-  }
-  const int dflt = dma_ok ? 0 : 1;
-  *idx = dflt;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  BH_HIP(hipStreamIsCapturing(stream(), &cs));
-  if (g_tune.mode == 0 || !repeatable || cs != hipStreamCaptureStatusNone) return BAMHIP_OK;
-  TuneEntry te;
-  te.choice = dflt;
+// times every admissible variant of one launch over the regions R
+static int time_launch(int launch, const Z4cPtrs &P, const RegionLists &R, const Z4cK &K, int *flag, bool dma_ok,
+                       bool pairs_ok, TuneEntry &te) {
+  const Variant *V = kVariants[launch];
   hipEvent_t a, b;
   BH_HIP(hipEventCreate(&a));
   BH_HIP(hipEventCreate(&b));
   double best = 1e300;
   int e = BAMHIP_OK;
   for (int v = 0; v < kMaxVariants && e == BAMHIP_OK; v++) {
-    te.ms[v] = -1.0;
     if ((V[v].dma && !dma_ok) || (V[v].pairs && !pairs_ok)) continue;
     if ((e = V[v].fn(P, R, K, flag, stream()))) break;
     BH_HIP(hipEventRecord(a, stream()));
@@ -762,20 +744,41 @@ static int choose_variant(int kind, const Z4cPtrs &P, const RegionLists &R, cons
     BH_HIP(hipEventSynchronize(b));
     float ms = 0.0f;
     BH_HIP(hipEventElapsedTime(&ms, a, b));
-    te.ms[v] = ms / 2.0;
-    if (te.ms[v] < best) {
-      best = te.ms[v];
-      te.choice = v;
+    te.ms[launch][v] = ms / 2.0;
+    if (te.ms[launch][v] < best) {
+      best = te.ms[launch][v];
+      te.choice[launch] = v;
     }
   }
   BH_HIP(hipEventDestroy(a));
   BH_HIP(hipEventDestroy(b));
-  if (e) return e;
-  g_tune.chosen[kind][sig] = te;
-  *idx = te.choice;
-  // the outputs come from the chosen variant, as in every later call
-  *done = true;
-  return V[te.choice].fn(P, R, K, flag, stream());
+  return e;
+}
+
+// The tuner's choices for a level's regions R (by launch): those kept, or (mode
+// 1, outside capture, repeatable launches) those found by timing all variants on
+// the library stream; *te stays null otherwise.
+static int tuned(const Z4cPtrs &P, const RegionLists R[kLaunches], const bool has[kLaunches], const Z4cK &K, int *flag,
+                 bool repeatable, bool dma_ok, bool pairs_ok, const TuneEntry **te) {
+  const std::string sig = region_signature(R[kBoth], dma_ok, pairs_ok);
+  auto it = g_tune.chosen.find(sig);
+  if (it == g_tune.chosen.end()) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    BH_HIP(hipStreamIsCapturing(stream(), &cs));
+    if (g_tune.mode == 0 || !repeatable || cs != hipStreamCaptureStatusNone) return BAMHIP_OK;
+    TuneEntry n;
+    for (int l = 0; l < kLaunches; l++) {
+      n.choice[l] = -1;
+      for (double &t : n.ms[l]) t = -1.0;
+      if (!has[l]) continue;
+      if (int e = time_launch(l, P, R[l], K, flag, dma_ok, pairs_ok, n)) return e;
+    }
+    n.one = has[kBoth] && n.ms[kBoth][n.choice[kBoth]] <=
+                              n.ms[kBulk][n.choice[kBulk]] + n.ms[kShell][n.choice[kShell]];
+    it = g_tune.chosen.emplace(sig, n).first;
+  }
+  *te = &it->second;
+  return BAMHIP_OK;
 }
 
 // The tile and edge kernels of one RHS evaluation (plain, addlinear or fused
@@ -823,35 +826,44 @@ static int run_rhs(bamhip_level *lev, const Z4cPtrs &P, const Z4cK &K, bool chec
     repeatable = true;
   }
   const bool dma_ok = (long)lev->npoints * 8 < (1L << 32);
-  const RegionLists RB = {{&T.bulk, nullptr, nullptr, nullptr}}, RS = {{nullptr, &T.sx, &T.sy, &T.sz}},
-                    RA = {{&T.bulk, &T.sx, &T.sy, &T.sz}};
-  const bool have_shell = !T.sx.empty() || !T.sy.empty() || !T.sz.empty();
-  int ib = -1, is = -1;
-  bool db = false, ds = false;
+  const RegionLists R[kLaunches] = {{{&T.bulk, nullptr, nullptr, nullptr}},
+                                    {{nullptr, &T.sx, &T.sy, &T.sz}},
+                                    {{&T.bulk, &T.sx, &T.sy, &T.sz}}};
+  const bool bulk = !T.bulk.empty(), shell = !T.sx.empty() || !T.sy.empty() || !T.sz.empty();
+  const bool has[kLaunches] = {bulk, shell, bulk && shell};
   // 16-byte units hold element pairs (x, x + 1) with x even in every box:
   // even box rows, box offsets and tile rows (first staged x = i0 - 3 even)
   bool pairs_ok = true;
   for (const auto *v : {&T.bulk, &T.sx, &T.sy, &T.sz})
     for (const Z4cGeo &G : *v) pairs_ok = pairs_ok && G.m % 2 == 0 && G.noffset % 2 == 0 && (G.lo[0] - HALO) % 2 == 0;
-  if (!T.bulk.empty() &&
-      (e = choose_variant(0, PT, RB, KT, lev->d_flag, repeatable, dma_ok, pairs_ok, &ib, &db)))
+  const TuneEntry *te = nullptr;
+  if (((bulk && g_tune.forced[kBulk] < 0) || (shell && g_tune.forced[kShell] < 0)) &&
+      (e = tuned(PT, R, has, KT, lev->d_flag, repeatable, dma_ok, pairs_ok, &te)))
     return e;
-  if (have_shell && (e = choose_variant(1, PT, RS, KT, lev->d_flag, repeatable, dma_ok, pairs_ok, &is, &ds)))
-    return e;
-  if (K.rk) db = ds = false;  // the tuner ran the plain RHS; the stage itself is still to run
-  if (ib >= 0 && is >= 0 && !db && !ds && g_tune.overlap && kVariants[0][ib].fn == kVariants[1][is].fn) {
-    // bulk and slabs staged the same way: one launch
-    TimerScope t("z4_rhs");
-    if ((e = kVariants[0][ib].fn(P, RA, K, lev->d_flag, stream()))) return e;
-  } else {
-    if (ib >= 0 && !db) {
-      TimerScope t("z4_rhs");
-      if ((e = kVariants[0][ib].fn(P, RB, K, lev->d_flag, stream()))) return e;
+  int v[kLaunches] = {-1, -1, -1};
+  for (int l : {kBulk, kShell}) {
+    if (!has[l]) continue;
+    v[l] = g_tune.forced[l];
+    if (v[l] < 0) {
+      v[l] = te ? te->choice[l] : dma_ok ? 0 : 1;
+      continue;
     }
-    if (is >= 0 && !ds) {
-      TimerScope t("z4_rhs_edge");
-      if ((e = kVariants[1][is].fn(P, RS, K, lev->d_flag, stream()))) return e;
-    }
+    if (kVariants[l][v[l]].dma && !dma_ok)
+      return set_error(BAMHIP_EINVAL, "z4c tile variant '%s' needs a level below 2^29 points", kVariants[l][v[l]].name);
+    if (kVariants[l][v[l]].pairs && !pairs_ok)
+      return set_error(BAMHIP_EINVAL, "z4c tile variant '%s' needs even box sizes and offsets", kVariants[l][v[l]].name);
+  }
+  if (has[kBoth] && g_tune.overlap) {
+    if (te && g_tune.forced[kBulk] < 0 && g_tune.forced[kShell] < 0)
+      v[kBoth] = te->one ? te->choice[kBoth] : -1;
+    else if (v[kBulk] == v[kShell])
+      v[kBoth] = v[kBulk];
+  }
+  if (v[kBoth] >= 0) v[kBulk] = v[kShell] = -1;
+  for (int l = 0; l < kLaunches; l++) {
+    if (v[l] < 0) continue;
+    TimerScope t(l == kShell ? "z4_rhs_edge" : "z4_rhs");
+    if ((e = kVariants[l][v[l]].fn(P, R[l], K, lev->d_flag, stream()))) return e;
   }
   if (check_finite) {
     int h = 0;
@@ -1011,8 +1023,7 @@ extern "C" int bamhip_z4c_set_xcd_map(int on) {
 }
 
 extern "C" int bamhip_z4c_tune_clear(void) {
-  bamhip::g_tune.chosen[0].clear();
-  bamhip::g_tune.chosen[1].clear();
+  bamhip::g_tune.chosen.clear();
   return BAMHIP_OK;
 }
 
@@ -1037,20 +1048,29 @@ extern "C" int bamhip_z4c_force_variant(int kind, int idx) {
 }
 
 extern "C" int bamhip_z4c_tune_report(char *buf, int len) {
+  using namespace bamhip;
   std::string s;
   char line[160];
-  for (int kind = 0; kind < 2; kind++)
-    for (const auto &kv : bamhip::g_tune.chosen[kind]) {
-      const bamhip::TuneEntry &te = kv.second;
-      snprintf(line, sizeof line, "%s <- %zu regions:", bamhip::kVariants[kind][te.choice].name,
-               (size_t)std::count(kv.first.begin(), kv.first.end(), ';'));
-      s += line;
-      for (int v = 0; v < bamhip::kMaxVariants; v++) {
-        snprintf(line, sizeof line, " %s=%.4fms", bamhip::kVariants[kind][v].name, te.ms[v]);
-        s += line;
+  for (const auto &kv : g_tune.chosen) {
+    const TuneEntry &te = kv.second;
+    // the launches of a line, the ones that run first
+    const std::vector<int> one = {kBoth}, two = {kBulk, kShell};
+    for (const auto *ls : te.one ? std::initializer_list<const std::vector<int> *>{&one, &two}
+                                 : std::initializer_list<const std::vector<int> *>{&two, &one}) {
+      std::string name, times;
+      for (int l : *ls) {
+        if (te.choice[l] < 0) continue;
+        name += (name.empty() ? "" : ", ") + std::string(kVariants[l][te.choice[l]].name);
+        for (int v = 0; v < kMaxVariants; v++) {
+          snprintf(line, sizeof line, " %s=%.4fms", kVariants[l][v].name, te.ms[l][v]);
+          times += line;
+        }
       }
-      s += '\n';
+      if (name.empty()) continue;
+      snprintf(line, sizeof line, " <- %zu regions:", (size_t)std::count(kv.first.begin(), kv.first.end(), ';'));
+      s += name + line + times + '\n';
     }
+  }
   if (buf && len > 0) {
     const int n = (int)std::min<size_t>(s.size(), (size_t)len - 1);
     memcpy(buf, s.data(), n);

@@ -164,14 +164,16 @@ int bamhip_z4c_rhs(bamhip_level *lev, const bamhip_z4c_params *par,
  * indices name the same one); all variants give bitwise the same RHS.  In
  * mode 1 (default) the first bamhip_z4c_rhs call on a new set of boxes,
  * outside graph capture and with unew not aliasing upre, times every variant
- * and keeps the fastest for that set; mode 0 uses variant 0.
+ * and keeps the fastest for that set; bulk and shell are timed apart and in
+ * one launch.  Mode 0 uses variant 0.
  * bamhip_z4c_force_variant(kind, i) pins variant i (-1: back to the tuner).
- * tune_report writes one line per tuned set with the time of each variant and
- * returns the length needed (with the NUL). */
+ * tune_report writes one line per tuned set with the time of each variant,
+ * two for a set with bulk and shell (the launches in use first), and returns
+ * the length needed (with the NUL). */
 int bamhip_z4c_tune_mode(int mode);
 /* on != 0 (default): the bulk and box-edge shell tiles of a level run in one
- * launch where both are staged the same way, else one after the other; returns
- * the old value */
+ * launch unless the tuner found two to be faster, or variants that differ are
+ * pinned; 0: one after the other.  Returns the old value */
 int bamhip_z4c_set_overlap(int on);
 /* on != 0 (default): the tile kernels number their tiles so that each of the
  * 8 XCDs (workgroup w runs on XCD w mod 8) takes one contiguous range of

@@ -355,3 +355,78 @@ def test_every_index_of_a_variant_can_be_pinned():
         B.force_variant(B.BULK, -1)
         B.force_variant(B.SHELL, -1)
     lev.free()
+
+
+@pytest.fixture(scope="module")
+def uneven():
+    """three boxes of even rows and offsets with 33 bulk and 44 slab tiles, numbers that 8 does not divide,
+    and 25 fields of operands for the update forms"""
+    h, rng = 0.2, np.random.default_rng(12)
+    boxes, us = [], []
+    for (m, n, o), x0 in (((20, 20, 20), (-1.9, -1.8, -2.0)), ((22, 17, 26), (2.3, -1.5, -2.4)),
+                          ((8, 13, 7), (-0.4, 2.6, 0.3))):
+        ob = O.make_box(m, n, o, *x0, h, skip=(1,) * 6)
+        u = puncture_z4c(grid(ob), masses=((1.0, (0.05, -0.02, 0.03)),))
+        u[19:22] = 0.1 * rng.standard_normal((3,) + u.shape[1:])
+        us.append(u.reshape(25, -1))
+        boxes.append(B.make_box(m, n, o, *x0, h, skip=(1,) * 6))
+    lev = B.Level(boxes, 175)
+    lev.enable(range(175))
+    lev.put_state(U, np.concatenate(us, axis=1))
+    rng = np.random.default_rng(13)
+    for lst in (P, ACC):
+        lev.put_state(lst, lev.get_state(U) + 0.01 * rng.standard_normal((25, lev.npoints)))
+    yield lev
+    lev.free()
+
+
+@pytest.mark.parametrize("form", ["rhs", "addlinear", (True, True), (True, False), (False, False), (False, True)])
+def test_launches_and_stagings_bitwise_equal(uneven, form):
+    """every staging, bulk and slabs in one launch or in two, tiles numbered by XCD or not: bitwise one result"""
+    lev, par, first = uneven, B.z4c_params(), None
+    try:
+        for bulk, shell in ((0, 2), (1, 1), (5, 4)):
+            B.force_variant(B.BULK, bulk)
+            B.force_variant(B.SHELL, shell)
+            assert B.variants(B.BULK)[bulk].split()[2:] == B.variants(B.SHELL)[shell].split()[2:]
+            for overlap in (True, False):
+                for xcd in (True, False):
+                    B.set_overlap(overlap)
+                    B.set_xcd_map(xcd)
+                    for v in R + A + V + CP:
+                        lev.fill(v, 0.0)
+                    if form == "rhs":
+                        lev.z4c_rhs(par, R, U)
+                    elif form == "addlinear":
+                        lev.z4c_rhs(par, R, U, upre=P, c=0.05)
+                    else:
+                        _stage(lev, par, U, ACC, A, P, V if form[0] else None, CP if form[1] else None, 0.3, 0.7)
+                    got = lev.get_state(R + A + V + CP)
+                    first = got if first is None else first
+                    np.testing.assert_array_equal(got, first, err_msg=str((bulk, overlap, xcd)))
+    finally:
+        B.force_variant(B.BULK, -1)
+        B.force_variant(B.SHELL, -1)
+        B.set_overlap(True)
+        B.set_xcd_map(True)
+    assert np.abs(first).max() > 0
+
+
+def test_tuner_times_the_launches_that_run(uneven):
+    """a level with bulk and shell: the fastest single launch against the fastest pair, the faster one first"""
+    B.tune_clear()
+    uneven.z4c_rhs(B.z4c_params(), R, U)
+    lines = B.tune_report().splitlines()
+    assert len(lines) == 2
+    cost, names = [], []
+    for line in lines:
+        name, times = line.split(" <- ")
+        ms = dict(t.rsplit("=", 1) for t in times.split(": ", 1)[1].removesuffix("ms").split("ms "))
+        picked = name.split(", ")
+        for p in picked:
+            same = [float(t) for n, t in ms.items() if n.split()[:2] == p.split()[:2]]
+            assert len(same) == 3 and float(ms[p]) == min(same)
+        cost.append(sum(float(ms[p]) for p in picked))
+        names.append(picked)
+    assert cost[0] <= cost[1]
+    assert sorted(len(n) for n in names) == [1, 2]
