@@ -648,6 +648,26 @@ int bamhip_vladd(bamhip_level *lev, int n, const int *r, double ca, const int *a
 
 }  // extern "C"
 
+// whether an output of the radiative condition is an operand or an output of
+// another variable, which runs in a block of its own
+static bool radiative_crossed(const Ptrs25 &N, const Ptrs25 &Pp, double c, const RkFuse &F) {
+  const double *const *out[3] = {N.p, F.uc.p, F.copy.p}, *const *in[2] = {Pp.p, F.ucin.p};
+  const bool has_out[3] = {!F.rk || F.has_v, F.rk != 0, F.rk && F.has_cp},
+             has_in[2] = {F.rk ? F.has_v || F.has_cp : c != 0.0, F.rk != 0};
+  for (int x = 0; x < 3; x++) {
+    if (!has_out[x]) continue;
+    for (int v = 0; v < 25; v++)
+      for (int w = 0; w < 25; w++) {
+        if (v == w) continue;
+        for (int y = 0; y < 2; y++)
+          if (has_in[y] && out[x][v] == in[y][w]) return true;
+        for (int y = x; y < 3; y++)
+          if (has_out[y] && out[x][v] == out[y][w]) return true;
+      }
+  }
+  return false;
+}
+
 // The boundary of one RHS evaluation or fused RK4 stage on every box:
 // radiative condition on PHYBOUND faces, periodic copy of pgh layers of the
 // lists in per_lists on PERBOUND face pairs.
@@ -661,19 +681,10 @@ static int boundary_impl(bamhip_level *lev, const bamhip_z4c_params *par, Ptrs25
     ri.var0[v] = (v == 0 || v == 3 || v == 5 || v == 6 || v == 18) ? 1.0 : 0.0;
     ri.v[v] = (v == 6 || v == 18 || v == 13) ? vg : 1.0;
   }
-  // variables run in blocks of their own: no order between an output and
-  // another variable's operands or outputs
-  const double *const *out[3] = {N.p, F.uc.p, F.copy.p}, *const *in[2] = {Pp.p, F.ucin.p};
-  const bool has_out[3] = {!F.rk || F.has_v, F.rk != 0, F.rk && F.has_cp},
-             has_in[2] = {F.rk ? F.has_v || F.has_cp : c != 0.0, F.rk != 0};
-  bool crossed = false;
-  for (int v = 0; v < 25; v++)
-    for (int w = 0; w < 25; w++)
-      for (int x = 0; x < 3; x++) {
-        if (v == w || !has_out[x]) continue;
-        for (int y = 0; y < 2; y++) crossed |= has_in[y] && out[x][v] == in[y][w];
-        for (int y = 0; y < 3; y++) crossed |= has_out[y] && out[x][v] == out[y][w];
-      }
+  bool radiative = false;
+  for (const DevBox &B : lev->boxes)
+    for (int f = 0; f < 6; f++) radiative |= B.bflag[f] == BAMHIP_PHYBOUND;
+  const bool crossed = radiative && radiative_crossed(N, Pp, c, F);
   TimerScope t("set_boundary");
   for (const DevBox &B : lev->boxes) {
     bool anyphy = false, anyper = false;
