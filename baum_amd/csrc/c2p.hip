@@ -516,9 +516,10 @@ __global__ void c2p_bracketed_hybrid_kernel(C2PArrays A, C2PK P, long n) {
 // features are not finite or whose polish does not converge falls back to
 // the cold-started bracketed solve (counted in *fallbacks).  The loop trip
 // count is uniform over the block, so every lane takes part in the network.
-// 4M points: 325 us with the activations through LDS and every load at its use;
-// 315 us with the activations in registers, 296 us with the next tile's inputs
-// loaded before the solve and the metric kept for the end (161 us of traffic).
+// 4M points under the profiler: 325 us with the activations through LDS and every
+// load at its use; 315 us with the activations in registers, 296 us with the next
+// tile's inputs loaded before the solve and the metric kept for the end.  Without
+// it the call went from 298 to 271 us (161 us of traffic).
 // Two waves per SIMD (229 registers): at three the network goes half the points
 // at a time, reads its weights twice, and takes 369 us.
 __global__ void __launch_bounds__(64) c2p_learned_kernel(C2PArrays A, C2PK P, MlpView M, long n, int polish_max,

@@ -930,9 +930,11 @@ static int check_params(const bamhip_z4c_params *par, const char *what) {
 // computed point accout = acc + wc RHS(src), when vout != NULL vout = base +
 // wv RHS(src), and when copy != NULL copy = base.  src is read by the
 // stencils, so no output may alias it; acc and base are read at the point
-// only, before any store, so an output may alias them (the accumulator read
-// from the list the next state goes to, for one).  The outputs must differ
-// from each other.  scratch (optional): 25 variables the tuner may use as a
+// only, so an output may alias them: of its own field in the tile kernel, which
+// reads a field's operands before it stores that field (the accumulator read
+// from the list the next state goes to, for one), of any field in the per-point
+// kernel, which takes such lists and reads all operands first.  The outputs must
+// differ from each other.  scratch (optional): 25 variables the tuner may use as a
 // plain RHS output the first time a box set is seen; it must not alias an
 // input (src, acc, base).
 int z4c_rhs_rk4_impl(bamhip_level *lev, const bamhip_z4c_params *par, const int *src, const int *acc,

@@ -331,8 +331,8 @@ constexpr int stage_nstores(int s) {
 // A wave's memory operations that may still be outstanding when it waits for
 // its transfers of stage s's field, with each field's transfers (nper
 // operations) issued `lead` stages ahead and `per` stores a result: the later
-// fields' transfers and the stores of the stages since.  Loads between them
-// are not counted, which only waits for more.
+// fields' transfers and the stores of the stages since.  Loads, and the reloads
+// of spilled registers, between them are not counted, which only waits for more.
 constexpr int stage_outstanding(int s, int lead, int nper, int per) {
   int n = 0;
   for (int t = s - lead + 1; t < s; t++) n += (t + lead < 25 ? nper : 0) + per * stage_nstores(t);
@@ -455,9 +455,8 @@ __device__ __forceinline__ void pin(double (&a)[N]) {
 }
 
 // Regions of one launch: index ranges [lo, hi] of boxes of a level (bulk
-// regions, or slabs of the box-edge shell), each with its box geometry, and
-// the first block of each region.  All boxes of a level are computed by one
-// launch per tile layout.
+// regions, and slabs of the box-edge shell), each with its box geometry, and
+// the first block of each region.
 // The grid spacing constants are common to the regions of one launch (one
 // level), so a region carries only integer geometry.
 constexpr int kMaxRegions = 32;
@@ -1082,8 +1081,12 @@ __device__ __forceinline__ void tile_body(double *tile, int r, int b) {
 // after another and ended the evaluation: 24^3 box 0.11 ms, 64^3 0.16 ms.)
 // The slab tiles come first, so that none is left to the end.  Two blocks per
 // CU: 80 KB of LDS and 256 registers each.  SLABS = false: bulk regions only, as
-// of a periodic box (the kernel of all four bodies spills 20 more registers:
-// 2.42 instead of 2.24 ms on 192^3).
+// of a periodic box.  All kernels but one spill: by the compiler's report the
+// bulk alone 6-12 registers with 16-byte units, 14-21 with dwords and 0-8 through
+// registers, the kernel of all four bodies 79-128, 444-495 and 221-260 (8% more
+// time on 192^3 when that ran a box without slabs).  The slab bodies hold the
+// point's 18 advection coefficients besides, the dword units 20 offsets.  A
+// reload ends in a wait for every transfer in flight.
 //
 // Workgroups are dispatched to the 8 XCDs round-robin (workgroup w to XCD w mod
 // 8), each XCD with its own L2.  With xcd set, each XCD takes one contiguous
@@ -1128,11 +1131,11 @@ inline bool same_spacing(const Z4cGeo &a, const Z4cGeo &b) {
   return a.h[0] == b.h[0] && a.h[1] == b.h[1] && a.h[2] == b.h[2];
 }
 
-// one launch per kMaxRegions regions of a layout (and per grid spacing)
 // regions of one level by layout: the bulk, and slabs normal to x, y and z
 struct RegionLists {
   const std::vector<Z4cGeo> *kind[4];  // null: none of that kind
 };
+// one launch for all of them, or one per kMaxRegions regions and grid spacing
 template <int NB, int VEC>
 int launch_tiles(const Z4cPtrs &F, const RegionLists &R, const Z4cK &K, int *flag, hipStream_t st) {
   struct Reg {

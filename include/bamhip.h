@@ -552,8 +552,9 @@ int bamhip_rk4_last_update(bamhip_level *lev, const int *uc, const int *r, doubl
  * periodic layers of accout and vout, and with fill_skip sets vout, copy and
  * (when it is another list than acc) accout to base at the other points no
  * RHS kernel computes.  No output may alias src or another output; acc and
- * base are read at the point only and may alias outputs (with fill_skip, base
- * only the output of its own field: the fill is done first).  scratch
+ * base are read at the point only and may alias outputs (those of another
+ * field take slower kernels, one thread a point for all fields; with fill_skip,
+ * base only the output of its own field: the fill is done first).  scratch
  * (optional, 25 indices, not an input): a list the tile-kernel tuner may
  * overwrite with a plain RHS the first time a set of boxes is seen.  With
  * fusion selected, bamhip_z4c_rk4_stages rotates uc, up, r and v through
