@@ -430,3 +430,28 @@ def test_tuner_times_the_launches_that_run(uneven):
         names.append(picked)
     assert cost[0] <= cost[1]
     assert sorted(len(n) for n in names) == [1, 2]
+
+
+def test_level_of_more_regions_than_a_launch_holds():
+    """six boxes are 42 regions, a launch holds 32: the slabs of five boxes and more, then the rest and the
+    bulk regions; bitwise each box by itself"""
+    size, h = (14, 12, 10), 0.2
+    us, boxes = [], []
+    for b in range(6):
+        ob = O.make_box(*size, 3.0 * b - 8.0, -0.7, -0.8, h, skip=(1,) * 6)
+        us.append(puncture_z4c(grid(ob), masses=((1.0, (0.05, -0.02, 0.03)),)).reshape(25, -1))
+        boxes.append(B.make_box(*size, ob.x0, ob.y0, ob.z0, h))
+
+    def rhs(bs, u):
+        lev = B.Level(bs, 50)
+        lev.enable(range(50))
+        for v in R:
+            lev.fill(v, 0.0)
+        lev.put_state(U, u)
+        lev.z4c_rhs(B.z4c_params(), R, U)
+        got = lev.get_state(R)
+        lev.free()
+        return got
+
+    apart = np.concatenate([rhs([b], u) for b, u in zip(boxes, us)], axis=1)
+    np.testing.assert_array_equal(rhs(boxes, np.concatenate(us, axis=1)), apart)
